@@ -28,6 +28,13 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
           "-I", os.path.join(ROOT, "include")]
 
 PRODUCT_SOURCES = ["kernels.hip", "fast.hip", "fast_nt.hip", "plan.cpp", "capi.cpp"]
+# line_kernel.hip holds one kernel per precision and class: (object, defines)
+LINE_CLASSES = 7
+LINE_OBJECTS = [("line_%s%d.o" % (name, c),
+                 ["-DPFFT_LINE_REAL=" + real, "-DPFFT_LINE_NAME=" + name,
+                  "-DPFFT_LINE_CLASS=%d" % c])
+                for real, name in (("double", "f64"), ("float", "f32"))
+                for c in range(LINE_CLASSES)]
 EMU_SOURCES = ["emu.cpp", "plan.cpp"]
 
 
@@ -54,6 +61,11 @@ def build(verbose=False):
         lang = ["-x", "hip"] if src.endswith(".hip") else []
         dev = DEVICE_FLAGS if src.endswith(".hip") else []
         jobs.append([HIPCC] + COMMON + dev + lang + ["-c", os.path.join(CSRC, src), "-o", obj])
+        objs.append(obj)
+    for name, defines in LINE_OBJECTS:
+        obj = os.path.join(LIB, name)
+        jobs.append([HIPCC] + COMMON + DEVICE_FLAGS + defines +
+                    ["-x", "hip", "-c", os.path.join(CSRC, "line_kernel.hip"), "-o", obj])
         objs.append(obj)
     # host emulator (tests only): host compilation of the same phase functions
     for src in EMU_SOURCES:

@@ -123,6 +123,40 @@ struct PassArgs {
   const void* fs_tw;      // fs_M-point twiddles
 };
 
+// ---- line pass (line_pass.hpp) -----------------------------------------------
+constexpr int kLinePoints = 16;        // points a thread holds
+constexpr int kLineStages = 6;         // radix stages (radices 2 .. 16)
+constexpr int kLineMaxThreads = 512;   // workgroup
+// How a line's points are read and written: complex FFT, r2c and c2r of even
+// and of odd length, the R2R kinds (input gathers, post-processing through
+// LDS), and a complex FFT that carries a spectral operator or the twiddle of
+// a four-step split.
+enum LineClass : int32_t {
+  LC_C2C = 0, LC_R2C = 1, LC_C2R = 2, LC_R2C_ODD = 3, LC_C2R_ODD = 4, LC_R2R = 5, LC_C2C_OP = 6
+};
+constexpr int kLineClasses = 7;
+
+// One Stockham stage: butterfly j = jq ns + jj of the line's nb = M / rad
+// takes points j + r nb to points jq ns rad + jj + r ns, ns the product of the
+// earlier radices.
+struct LineStage {
+  uint32_t rad, nb, ns;
+  uint32_t m_nb, m_ns;   // reciprocals of nb and ns (line_div)
+  uint32_t tw;           // its twiddles w_(ns rad)^(r jj) in LineArgs::tw, at (r - 1) ns + jj
+};
+
+struct LineArgs {
+  int32_t S;             // stages (0: the pass does not run as a line pass)
+  int32_t cls;           // LineClass
+  uint32_t threads;
+  uint32_t Tw, twlog;    // work lines of a full tile, a power of two
+  uint32_t pitch, sh;    // LDS line pitch (points); a pad slot after every 2^sh points
+  uint32_t m_half;       // reciprocal of M / 2 + 1
+  int32_t jf_in, jf_out; // contiguous side: neighbouring threads along the line
+  const void* tw;
+  LineStage st[kLineStages];
+};
+
 template <typename R>
 struct cpx {
   R re, im;

@@ -12,6 +12,7 @@
 
 #include "../../include/pfft.h"
 #include "generic_pass.hpp"
+#include "line_pass.hpp"
 #include "plan.hpp"
 
 using namespace pfft;
@@ -33,6 +34,72 @@ static void emu_pass(const PassPlan& pp, const PassArgs& a) {
     for (int s = 0; s < fft_steps(a); ++s)
       for (int t = 0; t < nthr; ++t) phase_fft_step<R>(a, c, s, t, nthr, lds.data());
     for (int t = 0; t < nthr; ++t) phase_post<R>(a, c, t, nthr, lds.data());
+  }
+}
+
+// The line pass: every thread's registers live across the barriers.
+template <typename R, int CLS>
+static void emu_line(const PassPlan& pp, const PassArgs& a, const LineArgs& b) {
+  const int nthr = (int)b.threads;
+  std::vector<char> store((size_t)pp.lds_bytes + 16);
+  char* lds = store.data() + (16 - (size_t)store.data() % 16) % 16;
+  cpx<R>* W = (cpx<R>*)lds;
+  std::vector<cpx<R>> regs((size_t)nthr * kLinePoints);
+  const bool direct = line_direct(CLS);
+  const LineOp<R> op(a);
+  for (int64_t tile = 0; tile < a.ntiles; ++tile) {
+    TileCtx c;
+    tile_init(a, tile, c);
+    int64_t m0;
+    const OpLine<R> o = a.op ? op_tile<R>(a, tile, &m0) : OpLine<R>{R(0), R(1)};
+    for (int s = 0; s < b.S; ++s) {
+      const bool fin = s == b.S - 1;
+      for (int t = 0; t < nthr; ++t) {
+        cpx<R>* v = &regs[(size_t)t * kLinePoints];
+        if (s == 0) {
+#define PFFT_F(RAD) line_first<R, CLS, RAD>(a, b, c, op, o, t, v)
+          PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
+#undef PFFT_F
+        } else {
+#define PFFT_F(RAD) line_get<R, RAD>(b, c, s, fin && direct && b.jf_out, t, v, W)
+          PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
+#undef PFFT_F
+        }
+      }
+      for (int t = 0; t < nthr; ++t) {
+        cpx<R>* v = &regs[(size_t)t * kLinePoints];
+        if (fin && direct) {
+#define PFFT_F(RAD) line_store<R, CLS, RAD>(a, b, c, op, o, t, v)
+          PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
+#undef PFFT_F
+        } else {
+#define PFFT_F(RAD) line_put<R, RAD>(a, b, c, s, fin, t, v, W)
+          PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
+#undef PFFT_F
+        }
+      }
+    }
+    if (!direct)
+      for (int t = 0; t < nthr; ++t) line_post<R, CLS>(a, b, c, t, lds);
+  }
+}
+
+template <typename R>
+static void emu_any(const Plan& p, const PassPlan& pp, const PassArgs& a) {
+  if (!pp.line.S) {
+    emu_pass<R>(pp, a);
+    return;
+  }
+  LineArgs b = pp.line;
+  b.tw = table_at(p, pp.line_tw_id, true);
+  switch (b.cls == LC_C2C && (a.op || a.fs_M) ? (int)LC_C2C_OP : b.cls) {
+    case LC_C2C: emu_line<R, LC_C2C>(pp, a, b); break;
+    case LC_R2C: emu_line<R, LC_R2C>(pp, a, b); break;
+    case LC_C2R: emu_line<R, LC_C2R>(pp, a, b); break;
+    case LC_R2C_ODD: emu_line<R, LC_R2C_ODD>(pp, a, b); break;
+    case LC_C2R_ODD: emu_line<R, LC_C2R_ODD>(pp, a, b); break;
+    case LC_R2R: emu_line<R, LC_R2R>(pp, a, b); break;
+    default: emu_line<R, LC_C2C_OP>(pp, a, b); break;
   }
 }
 
@@ -106,8 +173,8 @@ __attribute__((visibility("default"))) int pfft_emu_execute_op(pfft_emu_plan* h,
     a.tile_order = h->tile_order;
     a.tile_rev = h->tile_rev;
     if (i == op_pass) op_fill(p, dir, *op, op_side, a);
-    if (p.real_type == PFFT_F32) emu_pass<float>(pp, a);
-    else emu_pass<double>(pp, a);
+    if (p.real_type == PFFT_F32) emu_any<float>(p, pp, a);
+    else emu_any<double>(p, pp, a);
   }
   return PFFT_OK;
 }

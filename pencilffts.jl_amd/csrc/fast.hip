@@ -67,88 +67,6 @@ __device__ __forceinline__ void line_sync() {
   else __syncthreads();
 }
 
-// ---- forward small DFTs in registers ----------------------------------------
-template <typename R>
-__device__ __forceinline__ void dft16(C<R>* v) {
-  // 16 = 4 x 4: n = 4a + b, k = k1 + 4 k2
-  const R c1 = R(0.92387953251128675612818318939679);  // cos(pi/8)
-  const R s1 = R(0.38268343236508977172845998403040);  // sin(pi/8)
-  const R h = R(0.70710678118654752440084436210485);
-  C<R> y[16];
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    C<R> t[4] = {v[b], v[4 + b], v[8 + b], v[12 + b]};
-    dft4(t);
-#pragma unroll
-    for (int k1 = 0; k1 < 4; ++k1) y[4 * b + k1] = t[k1];
-  }
-  // twiddles w16^(b k1)
-  y[5] = mk(y[5].re * c1 + y[5].im * s1, y[5].im * c1 - y[5].re * s1);      // w^1
-  y[6] = mk((y[6].re + y[6].im) * h, (y[6].im - y[6].re) * h);              // w^2
-  y[7] = mk(y[7].re * s1 + y[7].im * c1, y[7].im * s1 - y[7].re * c1);      // w^3
-  y[9] = mk((y[9].re + y[9].im) * h, (y[9].im - y[9].re) * h);              // w^2
-  y[10] = mul_mi(y[10]);                                                    // w^4
-  y[11] = mk((y[11].im - y[11].re) * h, -(y[11].re + y[11].im) * h);        // w^6
-  y[13] = mk(y[13].re * s1 + y[13].im * c1, y[13].im * s1 - y[13].re * c1); // w^3
-  y[14] = mk((y[14].im - y[14].re) * h, -(y[14].re + y[14].im) * h);        // w^6
-  y[15] = mk(-y[15].re * c1 - y[15].im * s1, -y[15].im * c1 + y[15].re * s1); // w^9
-#pragma unroll
-  for (int k1 = 0; k1 < 4; ++k1) {
-    C<R> t[4] = {y[k1], y[4 + k1], y[8 + k1], y[12 + k1]};
-    dft4(t);
-#pragma unroll
-    for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = t[k2];
-  }
-}
-
-// Good-Thomas prime-factor DFT of N1 N2 points, N1 and N2 coprime: with the
-// index maps n = (N2 n1 + N1 n2) mod N and k = (N2 <1/N2 mod N1> k1 + N1 <1/N1
-// mod N2> k2) mod N it is N1 DFTs of N2 points, then N2 DFTs of N1 points,
-// with no twiddles; the maps are compile-time register renamings.
-constexpr int inv_mod(int a, int m) {
-  for (int x = 1; x < m; ++x)
-    if ((a * x) % m == 1) return x;
-  return 1;
-}
-template <typename R, int RAD>
-__device__ __forceinline__ void dft(C<R>* v);
-template <typename R, int N1, int N2>
-__device__ __forceinline__ void dft_pfa(C<R>* v) {
-  constexpr int N = N1 * N2;
-  constexpr int E1 = N2 * inv_mod(N2 % N1, N1), E2 = N1 * inv_mod(N1 % N2, N2);
-  C<R> t[N1][N2];
-#pragma unroll
-  for (int n1 = 0; n1 < N1; ++n1)
-#pragma unroll
-    for (int n2 = 0; n2 < N2; ++n2) t[n1][n2] = v[(N2 * n1 + N1 * n2) % N];
-#pragma unroll
-  for (int n1 = 0; n1 < N1; ++n1) dft<R, N2>(t[n1]);
-#pragma unroll
-  for (int k2 = 0; k2 < N2; ++k2) {
-    C<R> u[N1];
-#pragma unroll
-    for (int n1 = 0; n1 < N1; ++n1) u[n1] = t[n1][k2];
-    dft<R, N1>(u);
-#pragma unroll
-    for (int k1 = 0; k1 < N1; ++k1) v[(E1 * k1 + E2 * k2) % N] = u[k1];
-  }
-}
-
-template <typename R, int RAD>
-__device__ __forceinline__ void dft(C<R>* v) {
-  if constexpr (RAD == 2) dft2(v);
-  else if constexpr (RAD == 3) dft3(v);
-  else if constexpr (RAD == 4) dft4(v);
-  else if constexpr (RAD == 5) dft5(v);
-  else if constexpr (RAD == 8) dft8(v);
-  else if constexpr (RAD == 16) dft16(v);
-  else if constexpr (RAD == 6) dft_pfa<R, 2, 3>(v);
-  else if constexpr (RAD == 10) dft_pfa<R, 2, 5>(v);
-  else if constexpr (RAD == 12) dft_pfa<R, 4, 3>(v);
-  else if constexpr (RAD == 20) dft_pfa<R, 4, 5>(v);
-  else static_assert(RAD == 0, "no register DFT of this radix");
-}
-
 // ---- one Stockham stage over one line ------------------------------------------
 // Butterfly j (0 <= j < M/RAD) of a stage with Ns = product of earlier radices:
 //   inputs  x[j + (M/RAD) r] * w_M^(r (j mod Ns) M/(Ns RAD))

@@ -14,6 +14,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "dft.hpp"
 
 namespace pfft {
 
@@ -60,7 +61,8 @@ struct Digits {
 // that the butterflies' stride-RAD writes (and the stride-8 ones of the
 // second stage) spread over the LDS banks instead of hitting a few of them.
 // The line pitch Mp covers wp(Mw - 1) + 1 slots.
-PFFT_HD uint32_t wp(uint32_t k) { return k + (k >> 3); }
+// (The line pass pads after every 2^sh points.)
+PFFT_HD uint32_t wp(uint32_t k, uint32_t sh = 3) { return k + (k >> sh); }
 
 // Tile index -> (block b0 of T lines along line dim 0, linear index `rest`
 // over line dims 1..D-1).  Order 0 walks line dim 0 first (consecutive tiles
@@ -407,60 +409,6 @@ PFFT_HD void phase_pre(const PassArgs& a, const TileCtx& c, int tid, int nthr,
 //   v_r = src[j + r M/R] * w_M^(r (j mod Ns) M/(Ns R)),  y = DFT_R(v),
 //   dst[(j / Ns) Ns R + (j mod Ns) + r Ns] = y_r.
 // Backward stages use DFT_bwd(v) = conj(DFT_fwd(conj(v))).
-template <typename R>
-PFFT_HD void dft2(cpx<R>* v) {
-  const cpx<R> a = v[0], b = v[1];
-  v[0] = a + b; v[1] = a - b;
-}
-template <typename R>
-PFFT_HD void dft3(cpx<R>* v) {
-  const R c = R(-0.5), s = R(0.86602540378443864676372317075294);
-  const cpx<R> t = v[1] + v[2];
-  const cpx<R> d = v[1] - v[2];
-  const cpx<R> m = v[0] + scl(t, c);
-  const cpx<R> u = mk(d.im * s, -d.re * s);  // -i s d
-  v[0] = v[0] + t;
-  v[1] = m + u;
-  v[2] = m - u;
-}
-template <typename R>
-PFFT_HD void dft4(cpx<R>* v) {
-  const cpx<R> t0 = v[0] + v[2], t1 = v[0] - v[2];
-  const cpx<R> t2 = v[1] + v[3], t3 = mul_mi(v[1] - v[3]);
-  v[0] = t0 + t2; v[2] = t0 - t2; v[1] = t1 + t3; v[3] = t1 - t3;
-}
-template <typename R>
-PFFT_HD void dft5(cpx<R>* v) {
-  const R c1 = R(0.30901699437494742410229341718282);
-  const R c2 = R(-0.80901699437494742410229341718282);
-  const R s1 = R(0.95105651629515357211643933337938);
-  const R s2 = R(0.58778525229247312916870595463907);
-  const cpx<R> a0 = v[0];
-  const cpx<R> sa = v[1] + v[4], da = v[1] - v[4];
-  const cpx<R> sb = v[2] + v[3], db = v[2] - v[3];
-  const cpx<R> p1 = a0 + scl(sa, c1) + scl(sb, c2);
-  const cpx<R> p2 = a0 + scl(sa, c2) + scl(sb, c1);
-  const cpx<R> q1 = scl(da, s1) + scl(db, s2);   // times -i
-  const cpx<R> q2 = scl(da, s2) - scl(db, s1);   // times -i
-  v[0] = a0 + sa + sb;
-  v[1] = p1 + mul_mi(q1);
-  v[4] = p1 - mul_mi(q1);
-  v[2] = p2 + mul_mi(q2);
-  v[3] = p2 - mul_mi(q2);
-}
-template <typename R>
-PFFT_HD void dft8(cpx<R>* v) {
-  const R h = R(0.70710678118654752440084436210485);
-  cpx<R> b[4], c[4];
-  for (int r = 0; r < 4; ++r) { b[r] = v[r] + v[r + 4]; c[r] = v[r] - v[r + 4]; }
-  c[1] = mk((c[1].re + c[1].im) * h, (c[1].im - c[1].re) * h);   // * (1-i)/sqrt2
-  c[2] = mul_mi(c[2]);                                           // * -i
-  c[3] = mk((c[3].im - c[3].re) * h, -(c[3].re + c[3].im) * h);  // * (-1-i)/sqrt2
-  dft4(b); dft4(c);
-  v[0] = b[0]; v[2] = b[1]; v[4] = b[2]; v[6] = b[3];
-  v[1] = c[0]; v[3] = c[1]; v[5] = c[2]; v[7] = c[3];
-}
-
 template <typename R, int RAD>
 PFFT_HD void stage_fixed(const PassArgs& a, const TileCtx& c, int64_t Ns, int64_t fftM, bool bwd,
                          const cpx<R>* src, cpx<R>* dst, int tid, int nthr) {
@@ -743,16 +691,17 @@ PFFT_HD void phase_fft_step(const PassArgs& a, const TileCtx& c, int i, int tid,
 
 // ---- phase 4: post-process and store --------------------------------------
 template <typename R>
-PFFT_HD R post_real(const PassArgs& a, const cpx<R>* W, uint32_t w, int64_t k) {
+PFFT_HD R post_real(const PassArgs& a, const cpx<R>* W, uint32_t pitch, uint32_t sh, uint32_t w,
+                    int64_t k) {
   const cpx<R>* aux = (const cpx<R>*)a.aux;
-  const cpx<R>* L = W + w * a.Mp;
+  const cpx<R>* L = W + w * pitch;
   const int64_t n = a.n;
   switch (a.kind) {
-    case L_C2R_HALF: return (k & 1) ? L[wp((uint32_t)(k >> 1))].im : L[wp((uint32_t)(k >> 1))].re;
-    case L_C2R_FULL: return L[wp((uint32_t)(k))].re;
+    case L_C2R_HALF: return (k & 1) ? L[wp((uint32_t)(k >> 1), sh)].im : L[wp((uint32_t)(k >> 1), sh)].re;
+    case L_C2R_FULL: return L[wp((uint32_t)(k), sh)].re;
     case L_DCT1: {
       // real line w is part w & 1 of work line w >> 1
-      const cpx<R> z = (W + (w >> 1) * a.Mp)[wp((uint32_t)k)];
+      const cpx<R> z = (W + (w >> 1) * pitch)[wp((uint32_t)k, sh)];
       return (w & 1) ? z.im : z.re;
     }
     case L_DCT2:
@@ -760,23 +709,23 @@ PFFT_HD R post_real(const PassArgs& a, const cpx<R>* W, uint32_t w, int64_t k) {
       // real line w is part w & 1 of work line w >> 1: its transform from
       // Z_q and conj Z_{n-q} (q = k, or n - 1 - k for the DST), then
       // y = 2 Re(w_4n^q V_q)
-      const cpx<R>* Z = W + (w >> 1) * a.Mp;
+      const cpx<R>* Z = W + (w >> 1) * pitch;
       const int64_t q = a.kind == L_DST2 ? n - 1 - k : k;
-      const cpx<R> Zq = Z[wp((uint32_t)q)];
-      const cpx<R> Zn = conj(Z[wp((uint32_t)(q == 0 ? 0 : n - q))]);
+      const cpx<R> Zq = Z[wp((uint32_t)q, sh)];
+      const cpx<R> Zn = conj(Z[wp((uint32_t)(q == 0 ? 0 : n - q), sh)]);
       const cpx<R> V = (w & 1) ? scl(mul_mi(Zq - Zn), R(0.5)) : scl(Zq + Zn, R(0.5));
       return R(2) * (aux[q] * V).re;
     }
     case L_DCT3:
     case L_DST3: {
       const int64_t m = (k & 1) ? n - 1 - (k >> 1) : (k >> 1);
-      const cpx<R> z = (W + (w >> 1) * a.Mp)[wp((uint32_t)m)];
+      const cpx<R> z = (W + (w >> 1) * pitch)[wp((uint32_t)m, sh)];
       const R y = (w & 1) ? z.im : z.re;
       return (a.kind == L_DST3 && (k & 1)) ? -y : y;
     }
     case L_DCT4:
     case L_DST4: {
-      const cpx<R> z = aux[n + k] * L[wp((uint32_t)(k))];
+      const cpx<R> z = aux[n + k] * L[wp((uint32_t)(k), sh)];
       const R y = R(2) * z.re;
       return (a.kind == L_DST4 && (k & 1)) ? -y : y;
     }
@@ -785,21 +734,21 @@ PFFT_HD R post_real(const PassArgs& a, const cpx<R>* W, uint32_t w, int64_t k) {
       // y_2m = Re(conj(e_m) (W_m + W_{m+n/2})), y_{n-1-2m} = -Im(...)
       const int64_t h = n / 2;
       const int64_t m = (k & 1) ? h - 1 - (k >> 1) : (k >> 1);
-      const cpx<R> z = conj(aux[h + m]) * (L[wp((uint32_t)m)] + L[wp((uint32_t)(m + h))]);
+      const cpx<R> z = conj(aux[h + m]) * (L[wp((uint32_t)m, sh)] + L[wp((uint32_t)(m + h), sh)]);
       const R y = (k & 1) ? -z.im : z.re;
       return (a.kind == L_DST4H && (k & 1)) ? -y : y;
     }
     case L_DST1: {
       // the odd extension's transform F of (a + i b) is S_b - i S_a
-      const cpx<R> z = (W + (w >> 1) * a.Mp)[wp((uint32_t)(k + 1))];
+      const cpx<R> z = (W + (w >> 1) * pitch)[wp((uint32_t)(k + 1), sh)];
       return (w & 1) ? z.re : -z.im;
     }
     case L_DHT: {
       // the transform of real line w (part w & 1 of work line w >> 1) by the
       // Hermitian split, then Re - Im
-      const cpx<R>* Z = W + (w >> 1) * a.Mp;
-      const cpx<R> Zk = Z[wp((uint32_t)k)];
-      const cpx<R> Zn = conj(Z[wp((uint32_t)(k == 0 ? 0 : n - k))]);
+      const cpx<R>* Z = W + (w >> 1) * pitch;
+      const cpx<R> Zk = Z[wp((uint32_t)k, sh)];
+      const cpx<R> Zn = conj(Z[wp((uint32_t)(k == 0 ? 0 : n - k), sh)]);
       const cpx<R> V = (w & 1) ? scl(mul_mi(Zk - Zn), R(0.5)) : scl(Zk + Zn, R(0.5));
       return V.re - V.im;
     }
@@ -813,33 +762,31 @@ PFFT_HD R post_real(const PassArgs& a, const cpx<R>* W, uint32_t w, int64_t k) {
 PFFT_HD int herm_weight(int64_t k, int64_t n) { return (k == 0 || 2 * k == n) ? 1 : 2; }
 
 template <typename R>
-PFFT_HD cpx<R> post_cplx(const PassArgs& a, const cpx<R>* W, uint32_t w, int64_t k) {
-  const cpx<R>* L = W + w * a.Mp;
+PFFT_HD cpx<R> post_cplx(const PassArgs& a, const cpx<R>* W, uint32_t pitch, uint32_t sh,
+                         uint32_t w, int64_t k) {
+  const cpx<R>* L = W + w * pitch;
   cpx<R> y;
   if (a.kind == L_R2C_HALF) {
     const cpx<R>* aux = (const cpx<R>*)a.aux;
     const int64_t M = a.M;
-    const cpx<R> Z = L[wp((uint32_t)(k == M ? 0 : k))];
-    const cpx<R> Zc = conj(L[wp((uint32_t)(k == 0 ? 0 : M - k))]);
+    const cpx<R> Z = L[wp((uint32_t)(k == M ? 0 : k), sh)];
+    const cpx<R> Zc = conj(L[wp((uint32_t)(k == 0 ? 0 : M - k), sh)]);
     const cpx<R> E = scl(Z + Zc, R(0.5));
     const cpx<R> O = scl(mul_mi(Z - Zc), R(0.5));
     y = E + aux[k] * O;
   } else {
-    y = L[wp((uint32_t)(k))];  // C2C, R2C_FULL
+    y = L[wp((uint32_t)(k), sh)];  // C2C, R2C_FULL
   }
   if (a.adjoint && (a.kind == L_R2C_HALF || a.kind == L_R2C_FULL))
     y = scl(y, R(herm_weight(k, a.n)));
   return y;
 }
 
+// The output elements from the line FFTs in W (line pitch and padding as
+// given; raw: the untransformed tile of a copy).
 template <typename R>
-PFFT_HD void phase_post(const PassArgs& a, const TileCtx& c, int tid, int nthr,
-                        char* lds) {
-  // the line FFT's output: the buffer its last stage wrote (work buffer 0
-  // after the Bluestein form's two FFTs)
-  const cpx<R>* W =
-      (const cpx<R>*)(lds + ((a.bs_M == 0 && (a.nstages & 1)) ? a.lds_w1_off : 0));
-  const R* raw = (const R*)(lds + a.lds_w1_off);
+PFFT_HD void phase_store(const PassArgs& a, const TileCtx& c, const cpx<R>* W, const R* raw,
+                         uint32_t pitch, uint32_t sh, int tid, int nthr) {
   const uint32_t L = (uint32_t)a.L_out;
   const uint32_t Tact = (uint32_t)c.Tact;
   const uint32_t count = Tact * L;
@@ -853,8 +800,8 @@ PFFT_HD void phase_post(const PassArgs& a, const TileCtx& c, int tid, int nthr,
     if (a.out_cplx) {
       cpx<R> y;
       if (a.kind == L_COPY) y = raw_cplx(a, raw, t, k);
-      else if (a.r2r_cplx) y = mk(post_real(a, W, 2 * t, k), post_real(a, W, 2 * t + 1, k));
-      else y = post_cplx(a, W, t, k);
+      else if (a.r2r_cplx) y = mk(post_real(a, W, pitch, sh, 2 * t, k), post_real(a, W, pitch, sh, 2 * t + 1, k));
+      else y = post_cplx(a, W, pitch, sh, t, k);
       if (a.fs_M) {
         const cpx<R> w = ((const cpx<R>*)a.fs_tw)[(c.m0 + t) * k];
         y = y * (a.bwd ? conj(w) : w);
@@ -868,11 +815,21 @@ PFFT_HD void phase_post(const PassArgs& a, const TileCtx& c, int tid, int nthr,
       }
       ((cpx<R>*)a.out)[g] = y;
     } else {
-      R y = a.kind == L_COPY ? raw[t * a.raw_pitch + k] : post_real(a, W, t, k);
+      R y = a.kind == L_COPY ? raw[t * a.raw_pitch + k] : post_real(a, W, pitch, sh, t, k);
       if (a.do_scale) y = y * sc;
       ((R*)a.out)[g] = y;
     }
   }
+}
+
+template <typename R>
+PFFT_HD void phase_post(const PassArgs& a, const TileCtx& c, int tid, int nthr,
+                        char* lds) {
+  // the line FFT's output: the buffer its last stage wrote (work buffer 0
+  // after the Bluestein form's two FFTs)
+  const cpx<R>* W =
+      (const cpx<R>*)(lds + ((a.bs_M == 0 && (a.nstages & 1)) ? a.lds_w1_off : 0));
+  phase_store<R>(a, c, W, (const R*)(lds + a.lds_w1_off), (uint32_t)a.Mp, 3, tid, nthr);
 }
 
 }  // namespace pfft

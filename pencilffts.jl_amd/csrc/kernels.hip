@@ -78,10 +78,46 @@ static void launch_generic_t(const PassPlan& pp, const PassArgs& a, hipStream_t 
   else
     hipLaunchKernelGGL((k_generic<R, kBlockThreads, false>), g, b, lds, st, a);
 }
-static void launch_generic(const PassPlan& pp, int real_type, const PassArgs& a,
+// ---- line pass ------------------------------------------------------------------
+// its kernels, one object per precision and class (line_kernel.hip)
+#define PFFT_LINE_EACH(X) \
+  X(f32, 0) X(f32, 1) X(f32, 2) X(f32, 3) X(f32, 4) X(f32, 5) X(f32, 6) \
+  X(f64, 0) X(f64, 1) X(f64, 2) X(f64, 3) X(f64, 4) X(f64, 5) X(f64, 6)
+#define PFFT_X(t, c)                              \
+  int line_prepare_##t##c(const PassPlan& pp);    \
+  void line_launch_##t##c(const PassPlan& pp, const PassArgs& a, const LineArgs& b, hipStream_t st);
+PFFT_LINE_EACH(PFFT_X)
+#undef PFFT_X
+struct LineKernel {
+  int (*prepare)(const PassPlan&);
+  void (*launch)(const PassPlan&, const PassArgs&, const LineArgs&, hipStream_t);
+};
+static const LineKernel& line_kernel(int real_type, int cls) {
+#define PFFT_X(t, c) {line_prepare_##t##c, line_launch_##t##c},
+  static const LineKernel k[2 * kLineClasses] = {PFFT_LINE_EACH(PFFT_X)};
+#undef PFFT_X
+  return k[(real_type == PFFT_F32 ? 0 : kLineClasses) + cls];
+}
+// the attributes of the kernels a line pass may launch (with an operator too)
+static int line_prepare(const Plan& p, const PassPlan& pp) {
+  int r = line_kernel(p.real_type, pp.line.cls).prepare(pp);
+  if (!r && pp.line.cls == LC_C2C) r = line_kernel(p.real_type, LC_C2C_OP).prepare(pp);
+  return r;
+}
+
+// the general kernel of a pass: the line pass, or the phases of the generic one
+static void launch_generic(const Plan& p, const PassPlan& pp, const PassArgs& a,
                            hipStream_t st) {
-  if (real_type == PFFT_F32) launch_generic_t<float>(pp, a, st);
-  else launch_generic_t<double>(pp, a, st);
+  if (pp.line.S) {
+    LineArgs b = pp.line;
+    b.tw = table_at(p, pp.line_tw_id);
+    const int cls = b.cls == LC_C2C && (a.op || a.fs_M) ? (int)LC_C2C_OP : b.cls;
+    line_kernel(p.real_type, cls).launch(pp, a, b, st);
+  } else if (p.real_type == PFFT_F32) {
+    launch_generic_t<float>(pp, a, st);
+  } else {
+    launch_generic_t<double>(pp, a, st);
+  }
 }
 
 #define HIP_TRY(expr)                                                             \
@@ -227,7 +263,7 @@ static int launch_pass(const Plan& p, const PassPlan& pp, const void* src, void*
     a.scale = 1.0 / p.scale;
   }
   if (pp.variant == 0) {
-    launch_generic(pp, p.real_type, a, st);
+    launch_generic(p, pp, a, st);
     return PFFT_OK;
   }
   return fast_launch(pp, a, st);
@@ -235,6 +271,7 @@ static int launch_pass(const Plan& p, const PassPlan& pp, const void* src, void*
 
 static int prepare_pass(const Plan& p, const PassPlan& pp) {
   if (pp.variant != 0) return fast_prepare(pp);
+  if (pp.line.S) return line_prepare(p, pp);
   return set_lds_limit(generic_fn(p.real_type, pp), pp.lds_bytes);
 }
 
@@ -710,29 +747,42 @@ void tune_forget() {
   g_tune_cache.clear();
 }
 
+static void free_tables(Plan& p) {
+  if (p.table_mem) (void)hipFree(p.table_mem);
+  p.table_mem = nullptr;
+  for (Table& t : p.tables) t.dev = nullptr;
+}
+
 int device_prepare(Plan& p) {
   if (p.dev) return PFFT_OK;
   DeviceState* d = new DeviceState();
   // on failure the tables go too, so a later prepare starts clean
   auto abandon = [&](int code) {
     delete d;
-    for (Table& t : p.tables) {
-      if (t.dev) (void)hipFree(t.dev);
-      t.dev = nullptr;
-    }
+    free_tables(p);
     return code;
   };
   if (hipGetDevice(&d->device) != hipSuccess)
     return abandon(fail(PFFT_ERR_DEVICE, "no HIP device available"));
-  for (Table& t : p.tables) {
-    const size_t bytes = t.host.size();
-    hipError_t e = hipMalloc(&t.dev, bytes);
+  // the tables, each at a multiple of 256 bytes, in one allocation and one copy
+  size_t bytes = 0;
+  auto place = [](size_t n) { return (n + 255) / 256 * 256; };
+  for (const Table& t : p.tables) bytes += place(t.host.size());
+  if (bytes) {
+    std::vector<uint8_t> image(bytes);
+    hipError_t e = hipMalloc(&p.table_mem, bytes);
     if (e != hipSuccess) {
-      t.dev = nullptr;
+      p.table_mem = nullptr;
       return abandon(
           fail(PFFT_ERR_ALLOC, std::string("hipMalloc(tables): ") + hipGetErrorString(e)));
     }
-    e = hipMemcpy(t.dev, t.host.data(), bytes, hipMemcpyHostToDevice);
+    size_t at = 0;
+    for (Table& t : p.tables) {
+      std::copy(t.host.begin(), t.host.end(), image.begin() + at);
+      t.dev = (char*)p.table_mem + at;
+      at += place(t.host.size());
+    }
+    e = hipMemcpy(p.table_mem, image.data(), bytes, hipMemcpyHostToDevice);
     if (e != hipSuccess)
       return abandon(
           fail(PFFT_ERR_DEVICE, std::string("hipMemcpy(tables): ") + hipGetErrorString(e)));
@@ -741,11 +791,7 @@ int device_prepare(Plan& p) {
   if (r) return abandon(r);
   for (auto* list : {&p.fwd, &p.bwd}) {
     for (PassPlan& pp : *list) {
-      if (pp.variant == 0) {
-        r = set_lds_limit(generic_fn(p.real_type, pp), pp.lds_bytes);
-      } else {
-        r = fast_prepare(pp);
-      }
+      r = prepare_pass(p, pp);
       if (r) return abandon(r);
     }
   }
@@ -819,7 +865,8 @@ int device_pass_names(Plan& p, int dir, std::string* out) {
   for (size_t i = 0; i < passes.size(); ++i) {
     if (i) *out += ";";
     *out += passes[i].variant == 0
-                ? std::string(p.real_type == PFFT_F32 ? "k_generic<f32>" : "k_generic<f64>")
+                ? std::string(passes[i].line.S ? "k_line" : "k_generic") +
+                      (p.real_type == PFFT_F32 ? "<f32>" : "<f64>")
                 : std::string(fast_name(passes[i].variant));
     if (passes[i].variant == 0 && passes[i].args.bs_M)
       *out += "/bluestein" + std::to_string(passes[i].args.bs_M);
@@ -828,10 +875,7 @@ int device_pass_names(Plan& p, int dir, std::string* out) {
 }
 
 void device_release(Plan& p) {
-  for (Table& t : p.tables) {
-    if (t.dev) (void)hipFree(t.dev);
-    t.dev = nullptr;
-  }
+  free_tables(p);
   if (p.dev) {
     if (p.dev->work) (void)hipFree(p.dev->work);
     for (int i = 0; i < p.dev->n_ev; ++i) (void)hipEventDestroy(p.dev->ev[i]);
@@ -1091,7 +1135,7 @@ int device_execute(Plan& p, int dir, const void* in, void* out, void* work, size
     }
     a.adjoint = adjoint ? 1 : 0;
     if (pp.variant == 0) {
-      launch_generic(pp, p.real_type, a, stream);
+      launch_generic(p, pp, a, stream);
     } else {
       r = fast_launch(pp, a, stream);
       if (r) return r;

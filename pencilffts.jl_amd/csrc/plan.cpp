@@ -245,11 +245,16 @@ static void expm(int64_t num, int64_t den, double* re, double* im) {
   }
 }
 
-static int add_table(Plan& p, const std::string& key_unused, std::vector<double>&& vals) {
-  (void)key_unused;
+// the plan's table of that key, -1 if there is none yet
+static int find_table(const Plan& p, const std::string& key) {
   for (size_t i = 0; i < p.tables.size(); ++i)
-    if (p.tables[i].values == vals) return (int)i;
+    if (p.tables[i].key == key) return (int)i;
+  return -1;
+}
+
+static int add_table(Plan& p, const std::string& key, std::vector<double>&& vals) {
   Table t;
+  t.key = key;
   t.real_bytes = p.real_type == PFFT_F32 ? 4 : 8;
   t.values = std::move(vals);
   const size_t n = t.values.size();
@@ -265,9 +270,12 @@ static int add_table(Plan& p, const std::string& key_unused, std::vector<double>
 }
 
 static int twiddle_table(Plan& p, int64_t M) {
+  const std::string key = "tw" + std::to_string(M);
+  const int have = find_table(p, key);
+  if (have >= 0) return have;
   std::vector<double> v(2 * M);
   for (int64_t k = 0; k < M; ++k) expm(k, M, &v[2 * k], &v[2 * k + 1]);
-  return add_table(p, "tw", std::move(v));
+  return add_table(p, key, std::move(v));
 }
 
 // Tables of the Bluestein form of an M-point FFT convolved at Mb points:
@@ -293,6 +301,11 @@ static int64_t dif_bin(int64_t pos, int64_t Mb, const int32_t* rad, int ns) {
 
 static void bluestein_tables(Plan& p, int64_t M, int64_t Mb, const int32_t* rad, int ns,
                              int32_t* chirp_id, int32_t* bhat_id) {
+  std::string key = std::to_string(M) + ":" + std::to_string(Mb);
+  for (int i = 0; i < ns; ++i) key += "," + std::to_string(rad[i]);
+  *chirp_id = find_table(p, "bs_chirp" + key);
+  *bhat_id = find_table(p, "bs_bhat" + key);
+  if (*chirp_id >= 0 && *bhat_id >= 0) return;
   std::vector<double> ch(2 * M);
   for (int64_t j = 0; j < M; ++j) expm((j * j) % (2 * M), 2 * M, &ch[2 * j], &ch[2 * j + 1]);
   std::vector<long double> re(Mb, 0.0L), im(Mb, 0.0L);
@@ -328,8 +341,8 @@ static void bluestein_tables(Plan& p, int64_t M, int64_t Mb, const int32_t* rad,
     bh[2 * pos] = (double)(re[k] / (long double)Mb);
     bh[2 * pos + 1] = (double)(im[k] / (long double)Mb);
   }
-  *chirp_id = add_table(p, "bs_chirp", std::move(ch));
-  *bhat_id = add_table(p, "bs_bhat", std::move(bh));
+  *chirp_id = add_table(p, "bs_chirp" + key, std::move(ch));
+  *bhat_id = add_table(p, "bs_bhat" + key, std::move(bh));
 }
 
 // LDS pitch (complex slots) of a generic-pass work line of Mw points: one
@@ -433,7 +446,14 @@ static int line_fft(Plan& p, PassPlan& pp) {
     a.bs_M = Mb;
     bluestein_tables(p, M, Mb, a.radix, ns, &pp.bs_chirp_id, &pp.bs_bhat_id);
   }
-  // aux tables
+  // aux tables (one per kind family, n and M)
+  const int fam = lk == L_C2R_HALF ? L_R2C_HALF
+                  : lk == L_DST2 || lk == L_DCT3 || lk == L_DST3 ? L_DCT2
+                  : lk == L_DST4 ? L_DCT4 : lk == L_DST4H ? L_DCT4H : lk;
+  const std::string aux_key = "aux" + std::to_string(fam) + ":" + std::to_string(n) + ":" +
+                              std::to_string(M);
+  pp.aux_id = find_table(p, aux_key);
+  if (pp.aux_id >= 0) return PFFT_OK;
   std::vector<double> aux;
   if (lk == L_R2C_HALF || lk == L_C2R_HALF) {
     aux.resize(2 * (M + 1));
@@ -468,7 +488,7 @@ static int line_fft(Plan& p, PassPlan& pp) {
         expm(k2 * n1, 1024, &aux[2 * (64 * i + l)], &aux[2 * (64 * i + l) + 1]);
       }
   }
-  if (!aux.empty()) pp.aux_id = add_table(p, "aux", std::move(aux));
+  if (!aux.empty()) pp.aux_id = add_table(p, aux_key, std::move(aux));
   return PFFT_OK;
 }
 
@@ -478,6 +498,182 @@ struct LineDim {
   int64_t len, si, so;
   int logical;
 };
+
+// ---- line pass (line_pass.hpp) ------------------------------------------------
+static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Threads per line of a schedule: the stage with the most butterflies per
+// thread slot decides.
+static double line_load(int64_t M, const int32_t* rad, int ns) {
+  double worst = 0;
+  for (int s = 0; s < ns; ++s)
+    worst = std::max(worst, (double)(M / rad[s]) / (kLinePoints / rad[s]));
+  return worst;
+}
+
+// Radices of 2 to 16, descending, for an M-point line: the fewest stages (each
+// one more is another trip of the line through LDS), then the fewest threads
+// per line (a stage with fewer points per thread than the others leaves
+// threads idle).  0 where M does not factor that way.
+static int line_schedule(int64_t M, int32_t* best) {
+  int n_best = 0;
+  double load = 0;
+  int32_t cur[kLineStages];
+  auto rec = [&](auto&& self, int64_t m, int32_t top, int ns) -> void {
+    if (m == 1) {
+      const double l = line_load(M, cur, ns);
+      if (!n_best || ns < n_best || (ns == n_best && l < load)) {
+        n_best = ns;
+        load = l;
+        std::copy(cur, cur + ns, best);
+      }
+      return;
+    }
+    if (ns == kLineStages || (n_best && ns >= n_best)) return;
+    for (int32_t r = top; r >= 2; --r)
+      if (m % r == 0) {
+        cur[ns] = r;
+        self(self, m / r, r, ns + 1);
+      }
+  };
+  if (M > 1) rec(rec, M, 16, 0);
+  return n_best;
+}
+
+static uint32_t reciprocal(int64_t d) {
+  return d <= 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + d - 1) / d);
+}
+
+// Makes the generic form of a pass a line pass where it can be one: fills
+// pp.line, the tile, threads, LDS and twiddles.  A pass stays with the phases
+// of the generic kernel when it copies, when its FFT length has a prime
+// factor above 13 or runs as Bluestein, when one line takes more than
+// kLineMaxThreads threads (past about 8000 points) or the LDS, or when a lane's
+// offset within a tile would pass 2^31 bytes.
+static void line_setup(Plan& p, PassPlan& pp) {
+  PassArgs& a = pp.args;
+  LineArgs b = {};
+  if (a.kind == L_COPY || a.bs_M || a.M < 2) return;
+  int32_t rad[kLineStages];
+  const int S = line_schedule(a.M, rad);
+  if (!S) return;
+  b.S = S;
+  b.cls = a.kind == L_C2C        ? LC_C2C
+          : a.kind == L_R2C_HALF ? LC_R2C
+          : a.kind == L_C2R_HALF ? LC_C2R
+          : a.kind == L_R2C_FULL ? LC_R2C_ODD
+          : a.kind == L_C2R_FULL ? LC_C2R_ODD
+                                 : LC_R2R;
+  const int64_t rs = p.real_type == PFFT_F32 ? 4 : 8, cs = 2 * rs;
+  const bool direct = b.cls != LC_R2C && b.cls != LC_R2R;
+  b.jf_in = a.sk_in == 1;
+  b.jf_out = a.sk_out == 1;
+  // One pad slot per bank round (32 slots of 8 bytes, 16 of 16) spreads the
+  // even strides of the first stage's writes; the line pitch puts the lines
+  // of a tile side by side within a round, so that neighbouring threads on
+  // neighbouring lines, a butterfly apart, meet different banks.
+  b.sh = rs == 4 ? 5 : 4;
+  const int64_t round = rs == 4 ? 32 : 16;
+  const int64_t span = a.M + ((a.M - 1) >> b.sh);
+  auto lines = [&](int64_t T) {
+    const int64_t nreal = a.r2r_cplx ? 2 * T : T;
+    return a.pair_real ? (nreal + 1) / 2 : nreal;
+  };
+  auto pitch = [&](int64_t Tw) {
+    const int64_t want = Tw >= round ? 1 : round / Tw;
+    int64_t q = span;
+    while (q % round != want % round) ++q;
+    return q * 4 > span * 5 ? (span | 1) : q;   // short lines: odd will do
+  };
+  auto threads = [&](int64_t Tw) {
+    int64_t t = 0;
+    for (int s = 0; s < S; ++s)
+      t = std::max(t, ceil_div(Tw * (a.M / rad[s]), kLinePoints / rad[s]));
+    return ceil_div(t, 64) * 64;
+  };
+  auto bytes = [&](int64_t Tw) { return S == 1 && direct ? 0 : Tw * pitch(Tw) * cs; };
+  // lane offsets: 32 bits within a tile
+  auto reach = [&](int64_t T) {
+    const int64_t nb = a.M / rad[0], nbo = a.M / rad[S - 1];
+    const int64_t ein = a.in_cplx ? cs : rs, eout = a.out_cplx ? cs : rs;
+    const int64_t pin = b.cls == LC_R2C ? 2 : b.cls == LC_C2R_ODD ? rad[0] : 1;
+    const int64_t pout = b.cls == LC_C2R ? 2 : 1;
+    return std::max(((T - 1) * a.lsin[0] + pin * nb * a.sk_in) * ein,
+                    ((T - 1) * a.lsout[0] + pout * nbo * a.sk_out) * eout);
+  };
+  // Tile: 128-byte runs on a transposed side and about 256 threads; fewer
+  // lines where threads or LDS run out (two workgroups per CU at least), where
+  // the grid would not fill the chip, or where the last tile would be mostly
+  // empty.  Runs stay at 32 bytes or more.
+  const int64_t elt = (!b.jf_in && !a.in_cplx) || (!b.jf_out && !a.out_cplx) ? rs : cs;
+  const bool moved = !b.jf_in || !b.jf_out;
+  const int64_t run = moved ? 128 / elt : 1, run_min = moved ? 32 / elt : 1;
+  const int64_t least = a.pair_real && !a.r2r_cplx ? 2 : 1;
+  int64_t T = std::max(run, least);
+  while (T < 64 && threads(lines(T)) < 256) T *= 2;
+  int64_t cap = 1;
+  while (cap < a.ldim[0]) cap *= 2;
+  T = std::min(T, std::max(cap, least));
+  while (T > least && (threads(lines(T)) > kLineMaxThreads || bytes(lines(T)) > 80 * 1024)) T /= 2;
+  auto tiles = [&](int64_t t) {
+    int64_t n = ceil_div(a.ldim[0], t);
+    for (int i = 1; i < a.D; ++i) n *= a.ldim[i];
+    return n;
+  };
+  while (T > std::max(run_min, least) && T > least &&
+         (tiles(T) < 1024 || (a.ldim[0] * 5 < ceil_div(a.ldim[0], T) * T * 4)) &&
+         threads(lines(T)) > 64)
+    T /= 2;
+  const int64_t Tw = lines(T);
+  if (threads(Tw) > kLineMaxThreads || bytes(Tw) > kMaxLds || reach(T) >= ((int64_t)1 << 31)) return;
+  b.threads = (uint32_t)threads(Tw);
+  b.Tw = (uint32_t)Tw;
+  while (((int64_t)1 << b.twlog) < Tw) ++b.twlog;
+  b.pitch = (uint32_t)pitch(Tw);
+  b.m_half = reciprocal(a.M / 2 + 1);
+  // stages; their twiddles are entries of the M-point table, in the order the
+  // kernel reads them
+  std::string key = "line" + std::to_string(a.M);
+  int64_t ns = 1;
+  uint32_t entries = 0;
+  for (int s = 0; s < S; ++s) {
+    LineStage& st = b.st[s];
+    st.rad = (uint32_t)rad[s];
+    st.nb = (uint32_t)(a.M / rad[s]);
+    st.ns = (uint32_t)ns;
+    st.m_nb = reciprocal(st.nb);
+    st.m_ns = reciprocal(ns);
+    st.tw = entries;
+    if (s) entries += (uint32_t)((rad[s] - 1) * ns);
+    ns *= rad[s];
+    key += "," + std::to_string(rad[s]);
+  }
+  if (entries) {
+    pp.line_tw_id = find_table(p, key);
+    if (pp.line_tw_id < 0) {
+      const std::vector<double> w = p.tables[pp.tw_id].values;   // M points: not Bluestein
+      std::vector<double> tw;
+      tw.reserve(2 * entries);
+      for (int s = 1; s < S; ++s) {
+        const LineStage& st = b.st[s];
+        const int64_t step = a.M / ((int64_t)st.ns * st.rad);
+        for (int64_t r = 1; r < st.rad; ++r)
+          for (int64_t jj = 0; jj < st.ns; ++jj) {
+            const size_t k = 2 * (size_t)(r * jj * step);   // r jj < rad ns
+            tw.push_back(w[k]);
+            tw.push_back(w[k + 1]);
+          }
+      }
+      pp.line_tw_id = add_table(p, key, std::move(tw));
+    }
+  }
+  pp.line = b;
+  a.T = (int32_t)T;
+  pp.threads = (int32_t)b.threads;
+  pp.lds_bytes = bytes(Tw);
+  a.ntiles = tiles(T);
+  pp.grid = std::min<int64_t>(a.ntiles, 1 << 20);
+}
 
 // LDS budget of one generic-pass tile (the tile size T halves until it fits)
 #ifndef PFFT_GENERIC_TILE_LDS
@@ -574,6 +770,7 @@ static int line_layout(Plan& p, PassPlan& pp, std::vector<LineDim> lds, int dim,
   for (int i = 1; i < a.D; ++i) nt *= a.ldim[i];
   a.ntiles = nt;
   pp.grid = std::min<int64_t>(nt, 1 << 20);
+  line_setup(p, pp);
   a.scale = 1.0;
   a.do_scale = 0;
   pp.gen_args = a;
@@ -610,7 +807,7 @@ static int split_pass(Plan& p, const PassPlan& whole, const std::vector<LineDim>
   }
   PassPlan A = whole, B = whole;
   for (PassPlan* q : {&A, &B}) {
-    q->tw_id = q->aux_id = q->bs_chirp_id = q->bs_bhat_id = q->fs_tw_id = -1;
+    q->tw_id = q->aux_id = q->bs_chirp_id = q->bs_bhat_id = q->fs_tw_id = q->line_tw_id = -1;
     PassArgs& a = q->args;
     a.bs_M = 0;
     a.fs_M = 0;

@@ -60,13 +60,18 @@ struct PassPlan {
   int32_t gen_threads;
   int64_t gen_lds, gen_grid;
   int32_t variant_op = -1;  // operator-carrying variant (-1: not tuned, 0: generic)
+  // variant 0 as a line pass (line_pass.hpp) where line.S > 0, else the
+  // phases of the generic pass
+  LineArgs line = {};
+  int32_t line_tw_id = -1;  // index into Plan::tables (stage twiddles), -1 = none
 };
 
 struct Table {
+  std::string key;               // what it holds: passes of one plan share tables
   int32_t real_bytes;            // 4 or 8
   std::vector<double> values;    // interleaved re, im (double precision)
   std::vector<uint8_t> host;     // rounded to the plan's precision
-  void* dev = nullptr;           // device copy
+  void* dev = nullptr;           // device copy (within Plan::table_mem)
 };
 
 // ---- stage of the pencil chain ----------------------------------------------
@@ -102,15 +107,18 @@ struct Plan {
   std::vector<Table> tables;
   size_t in_bytes = 0, out_bytes = 0, work_bytes = 0, work0_bytes = 0;
   DeviceState* dev = nullptr;
+  void* table_mem = nullptr;   // one device allocation that holds every table
 };
 
-// Points a pass descriptor at the plan's tables: the device copies, or (host)
-// the copies rounded to the plan precision that the emulator reads.
+// A plan table: the device copy, or (host) the copy rounded to the plan
+// precision that the emulator reads; null for id -1.
+inline const void* table_at(const Plan& p, int32_t id, bool host = false) {
+  if (id < 0) return nullptr;
+  return host ? (const void*)p.tables[id].host.data() : (const void*)p.tables[id].dev;
+}
+// Points a pass descriptor at the plan's tables.
 inline void bind_tables(const Plan& p, const PassPlan& pp, PassArgs& a, bool host = false) {
-  auto at = [&](int32_t id) -> const void* {
-    if (id < 0) return nullptr;
-    return host ? (const void*)p.tables[id].host.data() : (const void*)p.tables[id].dev;
-  };
+  auto at = [&](int32_t id) { return table_at(p, id, host); };
   a.tw = at(pp.tw_id);
   a.aux = at(pp.aux_id);
   a.bs_chirp = at(pp.bs_chirp_id);
