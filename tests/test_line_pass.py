@@ -54,3 +54,15 @@ def test_line_pass_device(pf, gpu, dims, real_type, permute, extra):
             assert meta.kernels[0].startswith("k_line"), (name, meta.kernels)
         assert err_f <= tol and err_b <= tol, (name, err_f, err_b, tol)
 
+
+@pytest.mark.parametrize("dims", [(6, 9, 10), (9, 7, 8), (10, 9, 7), (7, 6, 9), (6, 5, 7, 8)],
+                         ids=lambda d: "x".join(map(str, d)))
+@pytest.mark.parametrize("kind", ["RFFT", "FFT"])
+def test_intermediate_orders(pf, emu, dims, kind):
+    """Odd and even extents in every place: the order of each intermediate is
+    chosen by them, and no choice may change the result."""
+    T = pf.Transforms
+    for rt in (1, 0):
+        tol = tol_for(CODE_NAMES[rt], dims)
+        err_f, err_b = emu_case(pf, emu, dims, (getattr(T, kind)(),), rt)
+        assert err_f <= tol and err_b <= tol, (err_f, err_b)
