@@ -28,13 +28,14 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
           "-I", os.path.join(ROOT, "include")]
 
 PRODUCT_SOURCES = ["kernels.hip", "fast.hip", "fast_nt.hip", "plan.cpp", "capi.cpp"]
-# line_kernel.hip holds one kernel per precision and class: (object, defines)
+# line_kernel.hip holds one kernel per precision, form (direct, Bluestein, prime
+# factors of 17 to 61) and class: (object, defines)
 LINE_CLASSES = 7
-LINE_OBJECTS = [("line_%s%d.o" % (name, c),
-                 ["-DPFFT_LINE_REAL=" + real, "-DPFFT_LINE_NAME=" + name,
-                  "-DPFFT_LINE_CLASS=%d" % c])
-                for real, name in (("double", "f64"), ("float", "f32"))
-                for c in range(LINE_CLASSES)]
+LINE_OBJECTS = [("line_%s_%s%d.o" % (name, form, c),
+                 ["-DPFFT_LINE_REAL=" + real, "-DPFFT_LINE_NAME=%s_%s" % (name, form),
+                  "-DPFFT_LINE_FORM=%d" % k, "-DPFFT_LINE_CLASS=%d" % c])
+                for c in reversed(range(LINE_CLASSES)) for k, form in enumerate(("", "bs", "prime"))
+                for real, name in (("double", "f64"), ("float", "f32"))]
 EMU_SOURCES = ["emu.cpp", "plan.cpp"]
 
 

@@ -107,10 +107,10 @@ struct PassArgs {
   double kmax[kMaxDims];    // per logical dim: largest stored |k|
   double op_alpha;
   // Bluestein (chirp-z) form of the M-point line FFT, for lengths with a
-  // large prime factor: X_k = c_k sum_j (x_j c_j) conj(c_{k-j}) with
-  // c_j = exp(-i pi j^2 / M), the convolution done by two bs_M-point FFTs
-  // (bs_M a power of two >= 2M - 1).  bs_M = 0: off.  With it, radix / nstages
-  // / tw describe the bs_M-point FFT.
+  // large prime factor (line_bluestein.hpp): X_k = c_k sum_j (x_j c_j)
+  // conj(c_{k-j}) with c_j = exp(-i pi j^2 / M), the convolution done by two
+  // bs_M-point FFTs (bs_M a power of two >= 2M - 1).  bs_M = 0:
+  // off.
   int64_t bs_M;
   const void* bs_chirp;   // c_j, j < M
   const void* bs_bhat;    // bs_M-point FFT of b_m = conj(c_m) (m mod bs_M, |m| < M), / bs_M,
@@ -125,7 +125,8 @@ struct PassArgs {
 
 // ---- line pass (line_pass.hpp) -----------------------------------------------
 constexpr int kLinePoints = 16;        // points a thread holds
-constexpr int kLineStages = 6;         // radix stages (radices 2 .. 16)
+constexpr int kLineStages = 6;         // radix stages (radices 2 .. 16, primes to 61)
+constexpr int kPrimePairs = 8;         // output pairs of a prime stage a thread keeps
 constexpr int kLineMaxThreads = 512;   // workgroup
 // How a line's points are read and written: complex FFT, r2c and c2r of even
 // and of odd length, the R2R kinds (input gathers, post-processing through
@@ -143,15 +144,25 @@ struct LineStage {
   uint32_t rad, nb, ns;
   uint32_t m_nb, m_ns;   // reciprocals of nb and ns (line_div)
   uint32_t tw;           // its twiddles w_(ns rad)^(r jj) in LineArgs::tw, at (r - 1) ns + jj
+                         // (a prime above 16: its roots w_rad^m first)
 };
+
+// How the line FFT is done (line_pass.hpp, line_bluestein.hpp, line_prime.hpp)
+enum LineForm : int32_t { LF_DIRECT = 0, LF_BLUESTEIN = 1, LF_PRIME = 2 };
+constexpr int kLineForms = 3;
+// Largest workgroup: float R2R kinds in the Bluestein form may need 8192 points
+// for each of two lines (the parts of complex data).
+constexpr int line_max_threads(int cls, int form, bool f32) {
+  return form == LF_BLUESTEIN && f32 && cls == LC_R2R ? 1024 : kLineMaxThreads;
+}
 
 struct LineArgs {
   int32_t S;             // stages (0: the pass does not run as a line pass)
-  int32_t cls;           // LineClass
+  int32_t cls, form;     // LineClass, LineForm
   uint32_t threads;
   uint32_t Tw, twlog;    // work lines of a full tile, a power of two
   uint32_t pitch, sh;    // LDS line pitch (points); a pad slot after every 2^sh points
-  uint32_t m_half;       // reciprocal of M / 2 + 1
+  uint32_t m_half, m_line;   // reciprocals of M / 2 + 1 and M
   int32_t jf_in, jf_out; // contiguous side: neighbouring threads along the line
   const void* tw;
   LineStage st[kLineStages];

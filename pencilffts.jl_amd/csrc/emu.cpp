@@ -12,7 +12,7 @@
 
 #include "../../include/pfft.h"
 #include "generic_pass.hpp"
-#include "line_pass.hpp"
+#include "line_prime.hpp"
 #include "plan.hpp"
 
 using namespace pfft;
@@ -31,8 +31,8 @@ static void emu_pass(const PassPlan& pp, const PassArgs& a) {
     tile_init(a, tile, c);
     for (int t = 0; t < nthr; ++t) phase_load<R>(a, c, t, nthr, lds.data());
     for (int t = 0; t < nthr; ++t) phase_pre<R>(a, c, t, nthr, lds.data());
-    for (int s = 0; s < fft_steps(a); ++s)
-      for (int t = 0; t < nthr; ++t) phase_fft_step<R>(a, c, s, t, nthr, lds.data());
+    for (int s = 0; s < a.nstages; ++s)
+      for (int t = 0; t < nthr; ++t) phase_stage<R>(a, c, s, t, nthr, lds.data());
     for (int t = 0; t < nthr; ++t) phase_post<R>(a, c, t, nthr, lds.data());
   }
 }
@@ -84,6 +84,91 @@ static void emu_line(const PassPlan& pp, const PassArgs& a, const LineArgs& b) {
   }
 }
 
+template <typename R, int CLS>
+static void emu_line_bs(const PassPlan& pp, const PassArgs& a, const LineArgs& b) {
+  const int nthr = (int)b.threads;
+  std::vector<char> store((size_t)pp.lds_bytes + 16);
+  char* lds = store.data() + (16 - (size_t)store.data() % 16) % 16;
+  cpx<R>* W = (cpx<R>*)lds;
+  const LineOp<R> op(a);
+  for (int64_t tile = 0; tile < a.ntiles; ++tile) {
+    TileCtx c;
+    tile_init(a, tile, c);
+    int64_t m0;
+    const OpLine<R> o = a.op ? op_tile<R>(a, tile, &m0) : OpLine<R>{R(0), R(1)};
+    for (int t = 0; t < nthr; ++t) {
+#define PFFT_F(RAD) bs_first<R, CLS, RAD>(a, b, c, op, o, t, W)
+      PFFT_LINE_RADIX(b.st[0].rad, PFFT_F)
+#undef PFFT_F
+    }
+    for (int i = 1; i < 2 * b.S - 2; ++i) {
+      const int s = i < b.S ? i : 2 * b.S - 2 - i;
+      const int dir = i < b.S - 1 ? 0 : i == b.S - 1 ? 1 : 2;
+      for (int t = 0; t < nthr; ++t) {
+#define PFFT_F(RAD) bs_stage<R, RAD>(a, b, c, s, dir, t, W)
+        PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
+#undef PFFT_F
+      }
+    }
+    for (int t = 0; t < nthr; ++t) {
+#define PFFT_F(RAD) bs_last<R, CLS, RAD>(a, b, c, op, o, t, W)
+      PFFT_LINE_RADIX(b.st[0].rad, PFFT_F)
+#undef PFFT_F
+    }
+    if (!line_direct(CLS))
+      for (int t = 0; t < nthr; ++t) line_post<R, CLS>(a, b, c, t, lds);
+  }
+}
+
+template <typename R, int CLS>
+static void emu_line_prime(const PassPlan& pp, const PassArgs& a, const LineArgs& b) {
+  const int nthr = (int)b.threads;
+  std::vector<char> store((size_t)pp.lds_bytes + 16);
+  char* lds = store.data() + (16 - (size_t)store.data() % 16) % 16;
+  cpx<R>* W = (cpx<R>*)lds;
+  std::vector<cpx<R>> regs((size_t)nthr * kLinePoints);
+  std::vector<PrimeRegs<R>> pregs((size_t)nthr);
+  const LineOp<R> op(a);
+  for (int64_t tile = 0; tile < a.ntiles; ++tile) {
+    TileCtx c;
+    tile_init(a, tile, c);
+    int64_t m0;
+    const OpLine<R> o = a.op ? op_tile<R>(a, tile, &m0) : OpLine<R>{R(0), R(1)};
+    for (int t = 0; t < nthr; ++t) prime_load<R, CLS>(a, b, c, op, o, t, W);
+    for (int s = 0; s < b.S; ++s) {
+      const bool fin = s == b.S - 1;
+      if (b.st[s].rad > 16) {
+        for (int t = 0; t < nthr; ++t) prime_get<R>(b, c, s, t, pregs[t], W);
+        for (int t = 0; t < nthr; ++t) prime_put<R>(a, b, c, s, fin, t, pregs[t], W);
+        continue;
+      }
+      for (int t = 0; t < nthr; ++t) {
+        cpx<R>* v = &regs[(size_t)t * kLinePoints];
+#define PFFT_F(RAD) line_get<R, RAD>(b, c, s, false, t, v, W)
+        PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
+#undef PFFT_F
+      }
+      for (int t = 0; t < nthr; ++t) {
+        cpx<R>* v = &regs[(size_t)t * kLinePoints];
+#define PFFT_F(RAD) line_put<R, RAD>(a, b, c, s, fin, t, v, W)
+        PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
+#undef PFFT_F
+      }
+    }
+    for (int t = 0; t < nthr; ++t) {
+      if constexpr (line_direct(CLS)) prime_save<R, CLS>(a, b, c, op, o, t, W);
+      else line_post<R, CLS>(a, b, c, t, lds);
+    }
+  }
+}
+
+template <typename R, int CLS>
+static void emu_form(const PassPlan& pp, const PassArgs& a, const LineArgs& b) {
+  if (b.form == LF_BLUESTEIN) emu_line_bs<R, CLS>(pp, a, b);
+  else if (b.form == LF_PRIME) emu_line_prime<R, CLS>(pp, a, b);
+  else emu_line<R, CLS>(pp, a, b);
+}
+
 template <typename R>
 static void emu_any(const Plan& p, const PassPlan& pp, const PassArgs& a) {
   if (!pp.line.S) {
@@ -93,13 +178,13 @@ static void emu_any(const Plan& p, const PassPlan& pp, const PassArgs& a) {
   LineArgs b = pp.line;
   b.tw = table_at(p, pp.line_tw_id, true);
   switch (b.cls == LC_C2C && (a.op || a.fs_M) ? (int)LC_C2C_OP : b.cls) {
-    case LC_C2C: emu_line<R, LC_C2C>(pp, a, b); break;
-    case LC_R2C: emu_line<R, LC_R2C>(pp, a, b); break;
-    case LC_C2R: emu_line<R, LC_C2R>(pp, a, b); break;
-    case LC_R2C_ODD: emu_line<R, LC_R2C_ODD>(pp, a, b); break;
-    case LC_C2R_ODD: emu_line<R, LC_C2R_ODD>(pp, a, b); break;
-    case LC_R2R: emu_line<R, LC_R2R>(pp, a, b); break;
-    default: emu_line<R, LC_C2C_OP>(pp, a, b); break;
+    case LC_C2C: emu_form<R, LC_C2C>(pp, a, b); break;
+    case LC_R2C: emu_form<R, LC_R2C>(pp, a, b); break;
+    case LC_C2R: emu_form<R, LC_C2R>(pp, a, b); break;
+    case LC_R2C_ODD: emu_form<R, LC_R2C_ODD>(pp, a, b); break;
+    case LC_C2R_ODD: emu_form<R, LC_C2R_ODD>(pp, a, b); break;
+    case LC_R2R: emu_form<R, LC_R2R>(pp, a, b); break;
+    default: emu_form<R, LC_C2C_OP>(pp, a, b); break;
   }
 }
 

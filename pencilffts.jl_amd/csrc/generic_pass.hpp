@@ -526,167 +526,33 @@ PFFT_HD void stage_any(const PassArgs& a, const TileCtx& c, int64_t Ns, int RAD,
   }
 }
 
-// Stage s of the line FFT (fftM points, radix schedule a.radix), from the
-// work buffer of parity sb to the other one; bwd: backward butterflies.
-// PRIME: radix 7, 11 and 13 as butterflies (stage_prime; its registers set
-// the kernel's, so only the instance for lines with such stages has it),
-// else as one work item per output (stage_any)
-template <typename R, bool PRIME = true>
-PFFT_HD void phase_stage_ex(const PassArgs& a, const TileCtx& c, int s, int sb, int64_t fftM,
-                            bool bwd, int tid, int nthr, char* lds) {
-  int64_t Ns = 1;
-  for (int i = 0; i < s; ++i) Ns *= a.radix[i];
-  const cpx<R>* src = (const cpx<R>*)(lds + ((sb & 1) ? a.lds_w1_off : 0));
-  cpx<R>* dst = (cpx<R>*)(lds + ((sb & 1) ? 0 : a.lds_w1_off));
-  switch (a.radix[s]) {
-    case 2: stage_fixed<R, 2>(a, c, Ns, fftM, bwd, src, dst, tid, nthr); break;
-    case 3: stage_fixed<R, 3>(a, c, Ns, fftM, bwd, src, dst, tid, nthr); break;
-    case 4: stage_fixed<R, 4>(a, c, Ns, fftM, bwd, src, dst, tid, nthr); break;
-    case 5: stage_fixed<R, 5>(a, c, Ns, fftM, bwd, src, dst, tid, nthr); break;
-    case 8: stage_fixed<R, 8>(a, c, Ns, fftM, bwd, src, dst, tid, nthr); break;
-    default:
-      if constexpr (PRIME) {
-        if (a.radix[s] == 7) { stage_prime<R, 7>(a, c, Ns, fftM, bwd, src, dst, tid, nthr); break; }
-        if (a.radix[s] == 11) { stage_prime<R, 11>(a, c, Ns, fftM, bwd, src, dst, tid, nthr); break; }
-        if (a.radix[s] == 13) { stage_prime<R, 13>(a, c, Ns, fftM, bwd, src, dst, tid, nthr); break; }
-      }
-      stage_any<R>(a, c, Ns, a.radix[s], fftM, bwd, src, dst, tid, nthr);
-      break;
-  }
-}
-
-// Stage s of the direct M-point line FFT.
+// Stage s of the M-point line FFT, from the work buffer of its parity to the
+// other one.  PRIME: radix 7, 11 and 13 as butterflies (stage_prime; its
+// registers set the kernel's, so only the instance for lines with such stages
+// has it), else as one work item per output (stage_any)
 template <typename R, bool PRIME = true>
 PFFT_HD void phase_stage(const PassArgs& a, const TileCtx& c, int s, int tid,
                          int nthr, char* lds) {
-  phase_stage_ex<R, PRIME>(a, c, s, s, a.M, a.bwd != 0, tid, nthr, lds);
-}
-
-// ---- Bluestein form of the line FFT ----------------------------------------
-// The M-point transform of the pre-processed lines in work buffer 0, all in
-// place there (one work buffer, so more workgroups fit on a CU):
-//   bs_pre   a_j = x_j c_j (x conjugated first for a backward transform),
-//            zero-padded to bs_M points;
-//   dif      the bs_M-point forward FFT, decimation in frequency over the
-//            radix schedule: bins land in digit-reversed positions;
-//   bs_mul   times the transform of b, stored in those positions (its
-//            1 / bs_M included);
-//   dit      the bs_M-point backward FFT, decimation in time over the
-//            stages in reverse: natural order again;
-//   bs_post  X_k = c_k C_k (conjugated back for a backward transform), k < M.
-//
-// In-place stage s of radix RAD over blocks of Bs = bs_M / (r_0 ... r_{s-1})
-// points: butterfly j < Bs / RAD of a block reads positions
-// j + q Bs / RAD (q < RAD).  Forward: DFT_RAD, then output q times
-// w_Bs^(q j).  Backward: input q times w_Bs^(-q j), then the conjugate DFT.
-template <typename R, int RAD>
-PFFT_HD void stage_inplace(const PassArgs& a, const TileCtx& c, int s, bool bwd, cpx<R>* W,
-                           int tid, int nthr) {
-  const cpx<R>* tw = (const cpx<R>*)a.tw;
-  const uint32_t Mb = (uint32_t)a.bs_M;
-  uint32_t Bs = Mb;
-  for (int i = 0; i < s; ++i) Bs /= (uint32_t)a.radix[i];
-  const uint32_t stride = Bs / RAD, tstep = Mb / Bs;
-  const uint32_t nb = Mb / RAD;                      // butterflies per line
-  const uint32_t count = (uint32_t)c.Tw * nb;
-  // e = (w (Mb / Bs) + blk) stride + j
-  Digits<3> it(tid, nthr, {stride, Mb / Bs});
-  for (uint32_t e = tid; e < count; e += nthr, it.next()) {
-    const uint32_t j = it.d[0], blk = it.d[1], w = it.d[2];
-    cpx<R>* L = W + w * a.Mp;
-    const uint32_t base = blk * Bs + j;
-    cpx<R> v[RAD];
-    for (int q = 0; q < RAD; ++q) {
-      v[q] = L[wp(base + q * stride)];
-      if (bwd) v[q] = conj(v[q]);
-      if (bwd && q) v[q] = v[q] * tw[q * j * tstep];   // conj(v w^-qj)
-    }
-    if (RAD == 2) dft2(v);
-    else if (RAD == 4) dft4(v);
-    else dft8(v);
-    for (int q = 0; q < RAD; ++q) {
-      cpx<R> y = v[q];
-      if (!bwd && q) y = y * tw[q * j * tstep];
-      L[wp(base + q * stride)] = bwd ? conj(y) : y;
-    }
-  }
-}
-
-template <typename R>
-PFFT_HD void phase_stage_inplace(const PassArgs& a, const TileCtx& c, int s, bool bwd, int tid,
-                                 int nthr, char* lds) {
-  cpx<R>* W = (cpx<R>*)lds;
+  int64_t Ns = 1;
+  for (int i = 0; i < s; ++i) Ns *= a.radix[i];
+  const bool bwd = a.bwd != 0;
+  const cpx<R>* src = (const cpx<R>*)(lds + ((s & 1) ? a.lds_w1_off : 0));
+  cpx<R>* dst = (cpx<R>*)(lds + ((s & 1) ? 0 : a.lds_w1_off));
   switch (a.radix[s]) {
-    case 2: stage_inplace<R, 2>(a, c, s, bwd, W, tid, nthr); break;
-    case 4: stage_inplace<R, 4>(a, c, s, bwd, W, tid, nthr); break;
-    default: stage_inplace<R, 8>(a, c, s, bwd, W, tid, nthr); break;
+    case 2: stage_fixed<R, 2>(a, c, Ns, a.M, bwd, src, dst, tid, nthr); break;
+    case 3: stage_fixed<R, 3>(a, c, Ns, a.M, bwd, src, dst, tid, nthr); break;
+    case 4: stage_fixed<R, 4>(a, c, Ns, a.M, bwd, src, dst, tid, nthr); break;
+    case 5: stage_fixed<R, 5>(a, c, Ns, a.M, bwd, src, dst, tid, nthr); break;
+    case 8: stage_fixed<R, 8>(a, c, Ns, a.M, bwd, src, dst, tid, nthr); break;
+    default:
+      if constexpr (PRIME) {
+        if (a.radix[s] == 7) { stage_prime<R, 7>(a, c, Ns, a.M, bwd, src, dst, tid, nthr); break; }
+        if (a.radix[s] == 11) { stage_prime<R, 11>(a, c, Ns, a.M, bwd, src, dst, tid, nthr); break; }
+        if (a.radix[s] == 13) { stage_prime<R, 13>(a, c, Ns, a.M, bwd, src, dst, tid, nthr); break; }
+      }
+      stage_any<R>(a, c, Ns, a.radix[s], a.M, bwd, src, dst, tid, nthr);
+      break;
   }
-}
-template <typename R>
-PFFT_HD void phase_bs_pre(const PassArgs& a, const TileCtx& c, int tid, int nthr, char* lds) {
-  cpx<R>* W = (cpx<R>*)lds;
-  const cpx<R>* ch = (const cpx<R>*)a.bs_chirp;
-  const uint32_t Mb = (uint32_t)a.bs_M, M = (uint32_t)a.M;
-  const uint32_t count = (uint32_t)c.Tw * Mb;
-  Digits<2> it(tid, nthr, {Mb});
-  for (uint32_t e = tid; e < count; e += nthr, it.next()) {
-    const uint32_t w = it.d[1], j = it.d[0];
-    cpx<R>* x = W + w * a.Mp + wp(j);
-    if (j < M) {
-      const cpx<R> v = a.bwd ? conj(*x) : *x;
-      *x = v * ch[j];
-    } else {
-      *x = mk(R(0), R(0));
-    }
-  }
-}
-
-template <typename R>
-PFFT_HD void phase_bs_mul(const PassArgs& a, const TileCtx& c, int tid, int nthr, char* lds) {
-  cpx<R>* W = (cpx<R>*)lds;
-  const cpx<R>* bh = (const cpx<R>*)a.bs_bhat;
-  const uint32_t Mb = (uint32_t)a.bs_M;
-  const uint32_t count = (uint32_t)c.Tw * Mb;
-  Digits<2> it(tid, nthr, {Mb});
-  for (uint32_t e = tid; e < count; e += nthr, it.next()) {
-    const uint32_t w = it.d[1], j = it.d[0];
-    cpx<R>* x = W + w * a.Mp + wp(j);
-    *x = *x * bh[j];
-  }
-}
-
-template <typename R>
-PFFT_HD void phase_bs_post(const PassArgs& a, const TileCtx& c, int tid, int nthr, char* lds) {
-  cpx<R>* W = (cpx<R>*)lds;
-  const cpx<R>* ch = (const cpx<R>*)a.bs_chirp;
-  const uint32_t M = (uint32_t)a.M;
-  const uint32_t count = (uint32_t)c.Tw * M;
-  Digits<2> it(tid, nthr, {M});
-  for (uint32_t e = tid; e < count; e += nthr, it.next()) {
-    const uint32_t w = it.d[1], k = it.d[0];
-    cpx<R>* x = W + w * a.Mp + wp(k);
-    const cpx<R> v = *x * ch[k];
-    *x = a.bwd ? conj(v) : v;
-  }
-}
-
-// ---- phase 3: the line FFT, as a sequence of barrier-separated steps -------
-// Direct form: the radix stages.  Bluestein form: bs_pre, the forward
-// stages, bs_mul, the backward stages, bs_post.
-PFFT_HD int fft_steps(const PassArgs& a) {
-  return a.bs_M ? 2 * a.nstages + 3 : a.nstages;
-}
-
-template <typename R, bool PRIME = true>
-PFFT_HD void phase_fft_step(const PassArgs& a, const TileCtx& c, int i, int tid, int nthr,
-                            char* lds) {
-  if (!a.bs_M) { phase_stage<R, PRIME>(a, c, i, tid, nthr, lds); return; }
-  const int ns = a.nstages;
-  if (i == 0) phase_bs_pre<R>(a, c, tid, nthr, lds);
-  else if (i <= ns) phase_stage_inplace<R>(a, c, i - 1, false, tid, nthr, lds);
-  else if (i == ns + 1) phase_bs_mul<R>(a, c, tid, nthr, lds);
-  else if (i <= 2 * ns + 1) phase_stage_inplace<R>(a, c, 2 * ns + 1 - i, true, tid, nthr, lds);
-  else phase_bs_post<R>(a, c, tid, nthr, lds);
 }
 
 // ---- phase 4: post-process and store --------------------------------------
@@ -825,10 +691,8 @@ PFFT_HD void phase_store(const PassArgs& a, const TileCtx& c, const cpx<R>* W, c
 template <typename R>
 PFFT_HD void phase_post(const PassArgs& a, const TileCtx& c, int tid, int nthr,
                         char* lds) {
-  // the line FFT's output: the buffer its last stage wrote (work buffer 0
-  // after the Bluestein form's two FFTs)
-  const cpx<R>* W =
-      (const cpx<R>*)(lds + ((a.bs_M == 0 && (a.nstages & 1)) ? a.lds_w1_off : 0));
+  // the line FFT's output: the buffer its last stage wrote
+  const cpx<R>* W = (const cpx<R>*)(lds + ((a.nstages & 1) ? a.lds_w1_off : 0));
   phase_store<R>(a, c, W, (const R*)(lds + a.lds_w1_off), (uint32_t)a.Mp, 3, tid, nthr);
 }
 

@@ -35,9 +35,8 @@ __global__ __launch_bounds__(NT) void k_generic(PassArgs a) {
       phase_pre<R>(a, c, threadIdx.x, blockDim.x, lds);
       __syncthreads();
     }
-    const int nsteps = fft_steps(a);
-    for (int s = 0; s < nsteps; ++s) {
-      phase_fft_step<R, PRIME>(a, c, s, threadIdx.x, blockDim.x, lds);
+    for (int s = 0; s < a.nstages; ++s) {
+      phase_stage<R, PRIME>(a, c, s, threadIdx.x, blockDim.x, lds);
       __syncthreads();
     }
     phase_post<R>(a, c, threadIdx.x, blockDim.x, lds);
@@ -47,7 +46,6 @@ __global__ __launch_bounds__(NT) void k_generic(PassArgs a) {
 
 // lines with a radix-7, 11 or 13 stage (the butterfly instance)
 static bool prime_stages(const PassArgs& a) {
-  if (a.bs_M) return false;
   for (int i = 0; i < a.nstages; ++i)
     if (a.radix[i] == 7 || a.radix[i] == 11 || a.radix[i] == 13) return true;
   return false;
@@ -79,10 +77,11 @@ static void launch_generic_t(const PassPlan& pp, const PassArgs& a, hipStream_t 
     hipLaunchKernelGGL((k_generic<R, kBlockThreads, false>), g, b, lds, st, a);
 }
 // ---- line pass ------------------------------------------------------------------
-// its kernels, one object per precision and class (line_kernel.hip)
-#define PFFT_LINE_EACH(X) \
-  X(f32, 0) X(f32, 1) X(f32, 2) X(f32, 3) X(f32, 4) X(f32, 5) X(f32, 6) \
-  X(f64, 0) X(f64, 1) X(f64, 2) X(f64, 3) X(f64, 4) X(f64, 5) X(f64, 6)
+// its kernels, one object per precision, form and class (line_kernel.hip)
+#define PFFT_LINE_SET(X, t) X(t, 0) X(t, 1) X(t, 2) X(t, 3) X(t, 4) X(t, 5) X(t, 6)
+#define PFFT_LINE_EACH(X)                                                          \
+  PFFT_LINE_SET(X, f32_) PFFT_LINE_SET(X, f32_bs) PFFT_LINE_SET(X, f32_prime)     \
+  PFFT_LINE_SET(X, f64_) PFFT_LINE_SET(X, f64_bs) PFFT_LINE_SET(X, f64_prime)
 #define PFFT_X(t, c)                              \
   int line_prepare_##t##c(const PassPlan& pp);    \
   void line_launch_##t##c(const PassPlan& pp, const PassArgs& a, const LineArgs& b, hipStream_t st);
@@ -92,16 +91,17 @@ struct LineKernel {
   int (*prepare)(const PassPlan&);
   void (*launch)(const PassPlan&, const PassArgs&, const LineArgs&, hipStream_t);
 };
-static const LineKernel& line_kernel(int real_type, int cls) {
+static const LineKernel& line_kernel(int real_type, int form, int cls) {
 #define PFFT_X(t, c) {line_prepare_##t##c, line_launch_##t##c},
-  static const LineKernel k[2 * kLineClasses] = {PFFT_LINE_EACH(PFFT_X)};
+  static const LineKernel k[2 * kLineForms * kLineClasses] = {PFFT_LINE_EACH(PFFT_X)};
 #undef PFFT_X
-  return k[(real_type == PFFT_F32 ? 0 : kLineClasses) + cls];
+  return k[((real_type == PFFT_F32 ? 0 : kLineForms) + form) * kLineClasses + cls];
 }
 // the attributes of the kernels a line pass may launch (with an operator too)
 static int line_prepare(const Plan& p, const PassPlan& pp) {
-  int r = line_kernel(p.real_type, pp.line.cls).prepare(pp);
-  if (!r && pp.line.cls == LC_C2C) r = line_kernel(p.real_type, LC_C2C_OP).prepare(pp);
+  const LineArgs& b = pp.line;
+  int r = line_kernel(p.real_type, b.form, b.cls).prepare(pp);
+  if (!r && b.cls == LC_C2C) r = line_kernel(p.real_type, b.form, LC_C2C_OP).prepare(pp);
   return r;
 }
 
@@ -112,7 +112,7 @@ static void launch_generic(const Plan& p, const PassPlan& pp, const PassArgs& a,
     LineArgs b = pp.line;
     b.tw = table_at(p, pp.line_tw_id);
     const int cls = b.cls == LC_C2C && (a.op || a.fs_M) ? (int)LC_C2C_OP : b.cls;
-    line_kernel(p.real_type, cls).launch(pp, a, b, st);
+    line_kernel(p.real_type, b.form, cls).launch(pp, a, b, st);
   } else if (p.real_type == PFFT_F32) {
     launch_generic_t<float>(pp, a, st);
   } else {

@@ -1,11 +1,12 @@
-// GPU kernel of the line pass (line_pass.hpp).  The file is compiled once per
-// precision (PFFT_LINE_REAL, PFFT_LINE_NAME) and class (PFFT_LINE_CLASS): each
+// GPU kernels of the line pass.  The file is compiled once per precision
+// (PFFT_LINE_REAL, PFFT_LINE_NAME), form (PFFT_LINE_FORM: line_pass.hpp,
+// line_bluestein.hpp or line_prime.hpp) and class (PFFT_LINE_CLASS): each
 // object holds one kernel with the butterflies of every radix.
 #include <hip/hip_runtime.h>
 
 #include <string>
 
-#include "line_pass.hpp"
+#include "line_prime.hpp"
 #include "plan.hpp"
 
 #define PFFT_CAT3_(a, b, c) a##b##c
@@ -22,6 +23,90 @@ __device__ __forceinline__ uint32_t opaque(uint32_t x) {
   return x;
 }
 
+#if PFFT_LINE_FORM == 1
+// (float: held to 128 VGPRs, 4 waves per SIMD; it asks for 130)
+template <typename R, int CLS>
+__global__ __launch_bounds__(line_max_threads(CLS, LF_BLUESTEIN, sizeof(R) == 4),
+                             sizeof(R) == 4 ? 4 : 2) void k_line_bs(PassArgs a, LineArgs b) {
+  extern __shared__ __align__(16) char lds[];
+  cpx<R>* W = (cpx<R>*)lds;
+  const uint32_t tid = threadIdx.x;
+  const LineOp<R> op(a);
+  for (int64_t tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x) {
+    TileCtx c;
+    tile_init(a, tile, c);
+    OpLine<R> o = {R(0), R(1)};
+    if constexpr (CLS == LC_C2C_OP) {
+      int64_t m0;
+      if (op.op) o = op_tile<R>(a, tile, &m0);
+    }
+#define PFFT_F(RAD) bs_first<R, CLS, RAD>(a, b, c, op, o, opaque(tid), W)
+    PFFT_LINE_RADIX(b.st[0].rad, PFFT_F)
+#undef PFFT_F
+    __syncthreads();
+    // forward stages 1 .. S-2, the middle one, backward S-2 .. 1
+    for (int i = 1; i < 2 * b.S - 2; ++i) {
+      const int s = i < b.S ? i : 2 * b.S - 2 - i;
+      const int dir = i < b.S - 1 ? 0 : i == b.S - 1 ? 1 : 2;
+#define PFFT_F(RAD) bs_stage<R, RAD>(a, b, c, s, dir, opaque(tid), W)
+      PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
+#undef PFFT_F
+      __syncthreads();
+    }
+#define PFFT_F(RAD) bs_last<R, CLS, RAD>(a, b, c, op, o, opaque(tid), W)
+    PFFT_LINE_RADIX(b.st[0].rad, PFFT_F)
+#undef PFFT_F
+    if constexpr (!line_direct(CLS)) {
+      __syncthreads();
+      line_post<R, CLS>(a, b, c, tid, lds);
+    }
+    __syncthreads();
+  }
+}
+#define PFFT_LINE_KERNEL k_line_bs
+#elif PFFT_LINE_FORM == 2
+template <typename R, int CLS>
+__global__ __launch_bounds__(kLineMaxThreads) void k_line_prime(PassArgs a, LineArgs b) {
+  extern __shared__ __align__(16) char lds[];
+  cpx<R>* W = (cpx<R>*)lds;
+  const uint32_t tid = threadIdx.x;
+  const LineOp<R> op(a);
+  for (int64_t tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x) {
+    TileCtx c;
+    tile_init(a, tile, c);
+    OpLine<R> o = {R(0), R(1)};
+    if constexpr (CLS == LC_C2C_OP) {
+      int64_t m0;
+      if (op.op) o = op_tile<R>(a, tile, &m0);
+    }
+    prime_load<R, CLS>(a, b, c, op, o, tid, W);
+    __syncthreads();
+    for (int s = 0; s < b.S; ++s) {
+      const bool fin = s == b.S - 1;
+      if (b.st[s].rad > 16) {
+        PrimeRegs<R> v;
+        prime_get<R>(b, c, s, tid, v, W);
+        __syncthreads();
+        prime_put<R>(a, b, c, s, fin, tid, v, W);
+      } else {
+        // (a prime came first: s > 0)
+        cpx<R> v[kLinePoints];
+#define PFFT_F(RAD)                                       \
+  line_get<R, RAD>(b, c, s, false, opaque(tid), v, W);    \
+  __syncthreads();                                        \
+  line_put<R, RAD>(a, b, c, s, fin, opaque(tid), v, W)
+        PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
+#undef PFFT_F
+      }
+      __syncthreads();
+    }
+    if constexpr (line_direct(CLS)) prime_save<R, CLS>(a, b, c, op, o, tid, W);
+    else line_post<R, CLS>(a, b, c, tid, lds);
+    __syncthreads();
+  }
+}
+#define PFFT_LINE_KERNEL k_line_prime
+#else
 template <typename R, int CLS>
 __global__ __launch_bounds__(kLineMaxThreads) void k_line(PassArgs a, LineArgs b) {
   extern __shared__ __align__(16) char lds[];
@@ -68,10 +153,13 @@ __global__ __launch_bounds__(kLineMaxThreads) void k_line(PassArgs a, LineArgs b
   }
 }
 
+#define PFFT_LINE_KERNEL k_line
+#endif
+
 int PFFT_CAT3(line_prepare_, PFFT_LINE_NAME, PFFT_LINE_CLASS)(const PassPlan& pp) {
   if (pp.lds_bytes <= 64 * 1024) return PFFT_OK;
   const hipError_t e =
-      hipFuncSetAttribute((const void*)k_line<PFFT_LINE_REAL, PFFT_LINE_CLASS>,
+      hipFuncSetAttribute((const void*)PFFT_LINE_KERNEL<PFFT_LINE_REAL, PFFT_LINE_CLASS>,
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)pp.lds_bytes);
   if (e != hipSuccess)
     return fail(PFFT_ERR_DEVICE, std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
@@ -81,8 +169,8 @@ int PFFT_CAT3(line_prepare_, PFFT_LINE_NAME, PFFT_LINE_CLASS)(const PassPlan& pp
 void PFFT_CAT3(line_launch_, PFFT_LINE_NAME, PFFT_LINE_CLASS)(const PassPlan& pp,
                                                               const PassArgs& a,
                                                               const LineArgs& b, hipStream_t st) {
-  hipLaunchKernelGGL((k_line<PFFT_LINE_REAL, PFFT_LINE_CLASS>), dim3((unsigned)pp.grid),
-                     dim3(b.threads), (size_t)pp.lds_bytes, st, a, b);
+  hipLaunchKernelGGL((PFFT_LINE_KERNEL<PFFT_LINE_REAL, PFFT_LINE_CLASS>),
+                     dim3((unsigned)pp.grid), dim3(b.threads), (size_t)pp.lds_bytes, st, a, b);
 }
 
 }  // namespace pfft

@@ -281,7 +281,7 @@ static int twiddle_table(Plan& p, int64_t M) {
 // Tables of the Bluestein form of an M-point FFT convolved at Mb points:
 // the chirp c_j = exp(-i pi j^2 / M), j < M (argument j^2 mod 2M reduced
 // exactly), and the Mb-point DFT of b_m = conj(c_|m|) (|m| < M, index m mod
-// Mb, zero elsewhere) divided by Mb, from a radix-2 FFT in long double.
+// Mb, zero elsewhere) divided by Mb, from an FFT in long double.
 // The kernel's forward convolution FFT runs in place, decimation in frequency
 // over the radix schedule rad[0..ns): its output position
 // p = q0 Mb/r0 + q1 Mb/(r0 r1) + ... holds bin q0 + r0 (q1 + r1 (q2 + ...)).
@@ -299,6 +299,35 @@ static int64_t dif_bin(int64_t pos, int64_t Mb, const int32_t* rad, int ns) {
   return k;
 }
 
+// Forward DFT in long double, by the smallest prime factor of the length.
+static std::vector<std::complex<long double>> fft_long(
+    const std::vector<std::complex<long double>>& x) {
+  using Z = std::complex<long double>;
+  const size_t n = x.size();
+  const long double tau = 6.283185307179586476925286766559005768L;
+  std::vector<Z> w(n), a = x, t(n);
+  for (size_t k = 0; k < n; ++k)
+    w[k] = {cosl(tau * (long double)k / (long double)n), -sinl(tau * (long double)k / (long double)n)};
+  // Stockham: ns points done, radix q
+  for (size_t ns = 1; ns < n;) {
+    size_t q = 2;
+    while ((n / ns) % q) ++q;
+    const size_t nb = n / q;
+    for (size_t j = 0; j < nb; ++j) {
+      const size_t jj = j % ns, o = j / ns * ns * q + jj;
+      for (size_t k = 0; k < q; ++k) {
+        Z acc = 0;
+        for (size_t r = 0; r < q; ++r)
+          acc += a[j + r * nb] * w[(r * jj * (nb / ns) + r * k % q * nb) % n];
+        t[o + k * ns] = acc;
+      }
+    }
+    std::swap(a, t);
+    ns *= q;
+  }
+  return a;
+}
+
 static void bluestein_tables(Plan& p, int64_t M, int64_t Mb, const int32_t* rad, int ns,
                              int32_t* chirp_id, int32_t* bhat_id) {
   std::string key = std::to_string(M) + ":" + std::to_string(Mb);
@@ -314,32 +343,14 @@ static void bluestein_tables(Plan& p, int64_t M, int64_t Mb, const int32_t* rad,
     im[m] = -(long double)ch[2 * m + 1];
     if (m) { re[Mb - m] = re[m]; im[Mb - m] = im[m]; }
   }
-  // in-place decimation-in-time FFT, bit-reversed input order
-  for (int64_t i = 1, j = 0; i < Mb; ++i) {
-    int64_t bit = Mb >> 1;
-    for (; j & bit; bit >>= 1) j ^= bit;
-    j ^= bit;
-    if (i < j) { std::swap(re[i], re[j]); std::swap(im[i], im[j]); }
-  }
-  const long double tau = 6.283185307179586476925286766559005768L;
-  for (int64_t len = 2; len <= Mb; len <<= 1) {
-    const int64_t h = len / 2;
-    for (int64_t k = 0; k < h; ++k) {
-      const long double wr = cosl(tau * (long double)k / (long double)len);
-      const long double wi = -sinl(tau * (long double)k / (long double)len);
-      for (int64_t s = 0; s < Mb; s += len) {
-        const int64_t u = s + k, v = s + k + h;
-        const long double tr = re[v] * wr - im[v] * wi, ti = re[v] * wi + im[v] * wr;
-        re[v] = re[u] - tr; im[v] = im[u] - ti;
-        re[u] += tr; im[u] += ti;
-      }
-    }
-  }
+  std::vector<std::complex<long double>> x(Mb);
+  for (int64_t m = 0; m < Mb; ++m) x[m] = {re[m], im[m]};
+  x = fft_long(x);
   std::vector<double> bh(2 * Mb);
   for (int64_t pos = 0; pos < Mb; ++pos) {
     const int64_t k = dif_bin(pos, Mb, rad, ns);
-    bh[2 * pos] = (double)(re[k] / (long double)Mb);
-    bh[2 * pos + 1] = (double)(im[k] / (long double)Mb);
+    bh[2 * pos] = (double)(x[k].real() / (long double)Mb);
+    bh[2 * pos + 1] = (double)(x[k].imag() / (long double)Mb);
   }
   *chirp_id = add_table(p, "bs_chirp" + key, std::move(ch));
   *bhat_id = add_table(p, "bs_bhat" + key, std::move(bh));
@@ -416,35 +427,114 @@ static void chain_perm(int N, int n, bool permute, int32_t* perm) {
   for (int i = n + 1; i < N; ++i) perm[i] = i;
 }
 
+// ---- line pass (line_pass.hpp) ------------------------------------------------
+static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Threads per line of a schedule: the stage with the most butterflies per
+// thread slot decides.
+static double line_load(int64_t M, const int32_t* rad, int ns) {
+  double worst = 0;
+  for (int s = 0; s < ns; ++s)
+    worst = std::max(worst, (double)(M / rad[s]) / (kLinePoints / rad[s]));
+  return worst;
+}
+
+// Radices of an M-point line: its prime factors of 17 to 61 first, then radices
+// of 2 to 16, descending: the fewest stages (each one more is another trip of
+// the line through LDS), then the fewest threads per line (a stage with fewer
+// points per thread than the others leaves threads idle).  0 where M does not
+// factor that way.
+static int line_schedule(int64_t M, int32_t* best) {
+  int primes = 0;
+  int64_t rest = M;
+  for (int32_t q : {61, 59, 53, 47, 43, 41, 37, 31, 29, 23, 19, 17})
+    while (rest % q == 0) {
+      if (primes == kLineStages) return 0;
+      best[primes++] = q;
+      rest /= q;
+    }
+  if (primes && rest == 1) return primes;
+  int n_best = 0;
+  double load = 0;
+  int32_t cur[kLineStages];
+  auto rec = [&](auto&& self, int64_t m, int32_t top, int ns) -> void {
+    if (m == 1) {
+      const double l = line_load(M, cur, ns);
+      if (!n_best || ns < n_best || (ns == n_best && l < load)) {
+        n_best = ns;
+        load = l;
+        std::copy(cur, cur + ns, best + primes);
+      }
+      return;
+    }
+    if (primes + ns == kLineStages || (n_best && ns >= n_best)) return;
+    for (int32_t r = top; r >= 2; --r)
+      if (m % r == 0) {
+        cur[ns] = r;
+        self(self, m / r, r, ns + 1);
+      }
+  };
+  if (M > 1) rec(rec, rest, 16, 0);
+  return n_best ? primes + n_best : 0;
+}
+
+static uint32_t reciprocal(int64_t d) {
+  return d <= 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + d - 1) / d);
+}
+
+static int line_class(int kind) {
+  return kind == L_C2C        ? LC_C2C
+         : kind == L_R2C_HALF ? LC_R2C
+         : kind == L_C2R_HALF ? LC_C2R
+         : kind == L_R2C_FULL ? LC_R2C_ODD
+         : kind == L_C2R_FULL ? LC_C2R_ODD
+                              : LC_R2R;
+}
+
+// Convolution length of the Bluestein form of an M-point line FFT, the power of
+// two at or above 2M - 1: 0 where M has no prime factor above kBluesteinPrime or
+// one line of the convolution does not fit the workgroup.
+static int64_t bluestein_length(const Plan& p, const PassArgs& a) {
+  const int64_t M = a.M;
+  if (largest_prime_factor(M) <= kBluesteinPrime) return 0;
+  int64_t Mb = 1;
+  while (Mb < 2 * M - 1) Mb *= 2;
+  // one line (two for the parts of complex data): the checks of line_setup
+  const int64_t Tw = a.r2r_cplx && !a.pair_real ? 2 : 1;
+  const bool f32 = p.real_type == PFFT_F32;
+  int32_t rad[kLineStages];
+  const int S = line_schedule(Mb, rad);
+  const int64_t points = Mb + (Mb >> (f32 ? 5 : 4)) + 32;
+  if (!S || Tw * points * (f32 ? 8 : 16) > kMaxLds ||
+      Tw * line_load(Mb, rad, S) > line_max_threads(line_class(a.kind), LF_BLUESTEIN, f32))
+    return 0;
+  return Mb;
+}
+
 // Build the pass for transforming logical dim `dim` from (perm_in, dims_in)
 // into (perm_out, dims_out).
 // Radix schedule, twiddles and per-kind tables of a pass's M-point line
-// FFT (a.kind, a.n, a.M, a.raw_pitch set).
-static int line_fft(Plan& p, PassPlan& pp) {
+// FFT (a.kind, a.n, a.M set); bluestein: in that form where it applies.
+static int line_fft(Plan& p, PassPlan& pp, bool bluestein = true) {
   PassArgs& a = pp.args;
   const int lk = a.kind;
   const int64_t M = a.M, n = a.n;
-  const int64_t rs = p.real_type == PFFT_F32 ? 4 : 8;
-  const int64_t cs = 2 * rs;
-  // A large prime factor makes the direct stages cost M p per line; the
-  // Bluestein form does the line in two FFTs of the next power of two at
-  // or above 2M - 1 instead, when one line of it fits the LDS.
-  int64_t Mb = 0;
-  if (largest_prime_factor(M) > kBluesteinPrime) {
-    Mb = 1;
-    while (Mb < 2 * M - 1) Mb *= 2;
-    // one work buffer (the convolution runs in place) beside the raw line
-    const int64_t Tw1 = a.r2r_cplx ? 2 : 1;
-    const int64_t w0 = (Tw1 * line_pitch_slots(Mb) * cs + 255) / 256 * 256;
-    if (w0 + a.raw_pitch * rs > kMaxLds) Mb = 0;
-  }
-  const int ns = radix_schedule(Mb ? Mb : M, a.radix);
-  if (ns < 0) return fail(PFFT_ERR_UNSUPPORTED, "too many radix stages");
-  a.nstages = ns;
-  pp.tw_id = twiddle_table(p, Mb ? Mb : M);
-  if (Mb) {
-    a.bs_M = Mb;
-    bluestein_tables(p, M, Mb, a.radix, ns, &pp.bs_chirp_id, &pp.bs_bhat_id);
+  // Two real R2R lines share one complex FFT as its real and imaginary
+  // parts: DCT-I / DST-I (real transforms), DCT-II / DST-II and DHT (split
+  // by Hermitian symmetry afterwards) and DCT-III / DST-III (Hermitian
+  // input, real transforms)
+  a.pair_real = (lk == L_DCT1 || lk == L_DST1 || lk == L_DCT2 || lk == L_DST2 ||
+                 lk == L_DCT3 || lk == L_DST3 || lk == L_DHT) ? 1 : 0;
+  a.bs_M = bluestein ? bluestein_length(p, a) : 0;
+  if (a.bs_M) {
+    int32_t rad[kLineStages];
+    const int S = line_schedule(a.bs_M, rad);
+    bluestein_tables(p, M, a.bs_M, rad, S, &pp.bs_chirp_id, &pp.bs_bhat_id);
+  } else {
+    const int ns = radix_schedule(M, a.radix);
+    if (ns < 0) return fail(PFFT_ERR_UNSUPPORTED, "too many radix stages");
+    a.nstages = ns;
+    pp.tw_id = twiddle_table(p, M);
   }
   // aux tables (one per kind family, n and M)
   const int fam = lk == L_C2R_HALF ? L_R2C_HALF
@@ -499,71 +589,25 @@ struct LineDim {
   int logical;
 };
 
-// ---- line pass (line_pass.hpp) ------------------------------------------------
-static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
-// Threads per line of a schedule: the stage with the most butterflies per
-// thread slot decides.
-static double line_load(int64_t M, const int32_t* rad, int ns) {
-  double worst = 0;
-  for (int s = 0; s < ns; ++s)
-    worst = std::max(worst, (double)(M / rad[s]) / (kLinePoints / rad[s]));
-  return worst;
-}
-
-// Radices of 2 to 16, descending, for an M-point line: the fewest stages (each
-// one more is another trip of the line through LDS), then the fewest threads
-// per line (a stage with fewer points per thread than the others leaves
-// threads idle).  0 where M does not factor that way.
-static int line_schedule(int64_t M, int32_t* best) {
-  int n_best = 0;
-  double load = 0;
-  int32_t cur[kLineStages];
-  auto rec = [&](auto&& self, int64_t m, int32_t top, int ns) -> void {
-    if (m == 1) {
-      const double l = line_load(M, cur, ns);
-      if (!n_best || ns < n_best || (ns == n_best && l < load)) {
-        n_best = ns;
-        load = l;
-        std::copy(cur, cur + ns, best);
-      }
-      return;
-    }
-    if (ns == kLineStages || (n_best && ns >= n_best)) return;
-    for (int32_t r = top; r >= 2; --r)
-      if (m % r == 0) {
-        cur[ns] = r;
-        self(self, m / r, r, ns + 1);
-      }
-  };
-  if (M > 1) rec(rec, M, 16, 0);
-  return n_best;
-}
-
-static uint32_t reciprocal(int64_t d) {
-  return d <= 1 ? 0u : (uint32_t)((((uint64_t)1 << 32) + d - 1) / d);
-}
-
 // Makes the generic form of a pass a line pass where it can be one: fills
 // pp.line, the tile, threads, LDS and twiddles.  A pass stays with the phases
 // of the generic kernel when it copies, when its FFT length has a prime
-// factor above 13 or runs as Bluestein, when one line takes more than
-// kLineMaxThreads threads (past about 8000 points) or the LDS, or when a lane's
-// offset within a tile would pass 2^31 bytes.
-static void line_setup(Plan& p, PassPlan& pp) {
+// factor above 61 whose convolution does not fit (bluestein_length), when one
+// line takes more than kLineMaxThreads threads (past about 8000 points) or
+// the LDS, or when a lane's offset within a tile would pass 2^31 bytes (the
+// other two forms' offsets are 64-bit).
+static bool line_setup(Plan& p, PassPlan& pp) {
   PassArgs& a = pp.args;
   LineArgs b = {};
-  if (a.kind == L_COPY || a.bs_M || a.M < 2) return;
+  if (a.kind == L_COPY || a.M < 2) return false;
+  const int64_t M = a.bs_M ? a.bs_M : a.M;   // points per work line
   int32_t rad[kLineStages];
-  const int S = line_schedule(a.M, rad);
-  if (!S) return;
+  const int S = line_schedule(M, rad);
+  if (!S) return false;
   b.S = S;
-  b.cls = a.kind == L_C2C        ? LC_C2C
-          : a.kind == L_R2C_HALF ? LC_R2C
-          : a.kind == L_C2R_HALF ? LC_C2R
-          : a.kind == L_R2C_FULL ? LC_R2C_ODD
-          : a.kind == L_C2R_FULL ? LC_C2R_ODD
-                                 : LC_R2R;
+  b.cls = line_class(a.kind);
+  b.form = a.bs_M ? LF_BLUESTEIN : rad[0] > 16 ? LF_PRIME : LF_DIRECT;
+  const int64_t max_threads = line_max_threads(b.cls, b.form, p.real_type == PFFT_F32);
   const int64_t rs = p.real_type == PFFT_F32 ? 4 : 8, cs = 2 * rs;
   const bool direct = b.cls != LC_R2C && b.cls != LC_R2R;
   b.jf_in = a.sk_in == 1;
@@ -574,7 +618,7 @@ static void line_setup(Plan& p, PassPlan& pp) {
   // neighbouring lines, a butterfly apart, meet different banks.
   b.sh = rs == 4 ? 5 : 4;
   const int64_t round = rs == 4 ? 32 : 16;
-  const int64_t span = a.M + ((a.M - 1) >> b.sh);
+  const int64_t span = M + ((M - 1) >> b.sh);
   auto lines = [&](int64_t T) {
     const int64_t nreal = a.r2r_cplx ? 2 * T : T;
     return a.pair_real ? (nreal + 1) / 2 : nreal;
@@ -587,14 +631,20 @@ static void line_setup(Plan& p, PassPlan& pp) {
   };
   auto threads = [&](int64_t Tw) {
     int64_t t = 0;
-    for (int s = 0; s < S; ++s)
-      t = std::max(t, ceil_div(Tw * (a.M / rad[s]), kLinePoints / rad[s]));
+    for (int s = 0; s < S; ++s) {
+      const int64_t n = Tw * (M / rad[s]);   // butterflies
+      t = std::max(t, rad[s] > 16 ? ceil_div(n, 64) * 64 * ceil_div((rad[s] - 1) / 2, kPrimePairs)
+                                  : ceil_div(n, kLinePoints / rad[s]));
+    }
     return ceil_div(t, 64) * 64;
   };
-  auto bytes = [&](int64_t Tw) { return S == 1 && direct ? 0 : Tw * pitch(Tw) * cs; };
+  auto bytes = [&](int64_t Tw) {
+    return S == 1 && direct && b.form == LF_DIRECT ? 0 : Tw * pitch(Tw) * cs;
+  };
   // lane offsets: 32 bits within a tile
-  auto reach = [&](int64_t T) {
-    const int64_t nb = a.M / rad[0], nbo = a.M / rad[S - 1];
+  auto reach = [&](int64_t T) -> int64_t {
+    if (b.form != LF_DIRECT) return 0;
+    const int64_t nb = M / rad[0], nbo = M / rad[S - 1];
     const int64_t ein = a.in_cplx ? cs : rs, eout = a.out_cplx ? cs : rs;
     const int64_t pin = b.cls == LC_R2C ? 2 : b.cls == LC_C2R_ODD ? rad[0] : 1;
     const int64_t pout = b.cls == LC_C2R ? 2 : 1;
@@ -614,7 +664,7 @@ static void line_setup(Plan& p, PassPlan& pp) {
   int64_t cap = 1;
   while (cap < a.ldim[0]) cap *= 2;
   T = std::min(T, std::max(cap, least));
-  while (T > least && (threads(lines(T)) > kLineMaxThreads || bytes(lines(T)) > 80 * 1024)) T /= 2;
+  while (T > least && (threads(lines(T)) > max_threads || bytes(lines(T)) > 80 * 1024)) T /= 2;
   auto tiles = [&](int64_t t) {
     int64_t n = ceil_div(a.ldim[0], t);
     for (int i = 1; i < a.D; ++i) n *= a.ldim[i];
@@ -625,38 +675,51 @@ static void line_setup(Plan& p, PassPlan& pp) {
          threads(lines(T)) > 64)
     T /= 2;
   const int64_t Tw = lines(T);
-  if (threads(Tw) > kLineMaxThreads || bytes(Tw) > kMaxLds || reach(T) >= ((int64_t)1 << 31)) return;
+  if (threads(Tw) > max_threads || bytes(Tw) > kMaxLds || reach(T) >= ((int64_t)1 << 31))
+    return false;
   b.threads = (uint32_t)threads(Tw);
   b.Tw = (uint32_t)Tw;
   while (((int64_t)1 << b.twlog) < Tw) ++b.twlog;
   b.pitch = (uint32_t)pitch(Tw);
   b.m_half = reciprocal(a.M / 2 + 1);
-  // stages; their twiddles are entries of the M-point table, in the order the
-  // kernel reads them
-  std::string key = "line" + std::to_string(a.M);
-  int64_t ns = 1;
+  b.m_line = reciprocal(a.M);
+  // Stages and their twiddles: entries of the M-point table in the order the
+  // kernel reads them (Bluestein: of the convolution's FFTs, decimation in
+  // frequency, ns the distance of a butterfly's points).
+  std::string key = (a.bs_M ? "bs_line" : "line") + std::to_string(M);
+  int64_t done = 1;
   uint32_t entries = 0;
   for (int s = 0; s < S; ++s) {
     LineStage& st = b.st[s];
     st.rad = (uint32_t)rad[s];
-    st.nb = (uint32_t)(a.M / rad[s]);
-    st.ns = (uint32_t)ns;
+    st.nb = (uint32_t)(M / rad[s]);
+    st.ns = (uint32_t)(a.bs_M ? M / (done * rad[s]) : done);
     st.m_nb = reciprocal(st.nb);
-    st.m_ns = reciprocal(ns);
+    st.m_ns = reciprocal(st.ns);
     st.tw = entries;
-    if (s) entries += (uint32_t)((rad[s] - 1) * ns);
-    ns *= rad[s];
+    if (rad[s] > 16) entries += (uint32_t)rad[s];   // its roots
+    if (a.bs_M ? s < S - 1 : s > 0) entries += (uint32_t)((rad[s] - 1) * st.ns);
+    done *= rad[s];
     key += "," + std::to_string(rad[s]);
   }
   if (entries) {
     pp.line_tw_id = find_table(p, key);
     if (pp.line_tw_id < 0) {
-      const std::vector<double> w = p.tables[pp.tw_id].values;   // M points: not Bluestein
+      std::vector<double> w(2 * M);
+      if (!a.bs_M) w = p.tables[pp.tw_id].values;
+      else
+        for (int64_t k = 0; k < M; ++k) expm(k, M, &w[2 * k], &w[2 * k + 1]);
       std::vector<double> tw;
       tw.reserve(2 * entries);
-      for (int s = 1; s < S; ++s) {
+      for (int s = 0; s < S; ++s) {
         const LineStage& st = b.st[s];
-        const int64_t step = a.M / ((int64_t)st.ns * st.rad);
+        if (st.rad > 16)
+          for (int64_t m = 0; m < st.rad; ++m) {
+            tw.push_back(w[2 * m * st.nb]);
+            tw.push_back(w[2 * m * st.nb + 1]);
+          }
+        if (a.bs_M ? s == S - 1 : s == 0) continue;
+        const int64_t step = M / ((int64_t)st.ns * st.rad);
         for (int64_t r = 1; r < st.rad; ++r)
           for (int64_t jj = 0; jj < st.ns; ++jj) {
             const size_t k = 2 * (size_t)(r * jj * step);   // r jj < rad ns
@@ -673,6 +736,7 @@ static void line_setup(Plan& p, PassPlan& pp) {
   pp.lds_bytes = bytes(Tw);
   a.ntiles = tiles(T);
   pp.grid = std::min<int64_t>(a.ntiles, 1 << 20);
+  return true;
 }
 
 // LDS budget of one generic-pass tile (the tile size T halves until it fits)
@@ -722,24 +786,31 @@ static int line_layout(Plan& p, PassPlan& pp, std::vector<LineDim> lds, int dim,
   }
   a.pdim = dim;
 
+  a.scale = 1.0;
+  a.do_scale = 0;
+  auto keep_generic = [&]() {
+    pp.gen_args = a;
+    pp.gen_threads = pp.threads;
+    pp.gen_lds = pp.lds_bytes;
+    pp.gen_grid = pp.grid;
+    return PFFT_OK;
+  };
+  if (line_setup(p, pp)) return keep_generic();
+  if (a.bs_M) {   // (no line pass after all: direct stages)
+    pp.bs_chirp_id = pp.bs_bhat_id = -1;
+    const int r = line_fft(p, pp, false);
+    if (r) return r;
+  }
   // tile size and LDS footprint of the generic pass
-  const int64_t Mw = a.bs_M ? a.bs_M : M;  // points per work line
-  a.Mp = line_pitch_slots(Mw);
+  a.Mp = line_pitch_slots(M);
   // c2c lines (and the real pairs of an even r2c, the Hermitian merge of an
   // even c2r) load straight into the work lines: no raw tile, no pre phase
   a.load_w0 = (lk == L_C2C || lk == L_R2C_HALF || lk == L_C2R_HALF) ? 1 : 0;
-  // Two real R2R lines share one complex FFT as its real and imaginary
-  // parts: DCT-I / DST-I (real transforms), DCT-II / DST-II and DHT (split
-  // by Hermitian symmetry afterwards) and DCT-III / DST-III (Hermitian
-  // input, real transforms)
-  a.pair_real = (lk == L_DCT1 || lk == L_DST1 || lk == L_DCT2 || lk == L_DST2 ||
-                 lk == L_DCT3 || lk == L_DST3 || lk == L_DHT) ? 1 : 0;
   auto footprint = [&](int64_t T, int64_t* w1off) {
     const int64_t nreal = a.r2r_cplx ? 2 * T : T;
     const int64_t Tw = a.pair_real ? (nreal + 1) / 2 : nreal;
     const int64_t w0 = lk == L_COPY ? 0 : Tw * a.Mp * cs;
-    // (the Bluestein form's convolution runs in place in work buffer 0)
-    const int64_t w1 = (lk == L_COPY || a.nstages == 0 || a.bs_M) ? 0 : Tw * a.Mp * cs;
+    const int64_t w1 = (lk == L_COPY || a.nstages == 0) ? 0 : Tw * a.Mp * cs;
     const int64_t raw = a.load_w0 ? 0 : T * a.raw_pitch * rs;
     *w1off = (w0 + 255) / 256 * 256;
     return *w1off + std::max(w1, raw);
@@ -759,25 +830,18 @@ static int line_layout(Plan& p, PassPlan& pp, std::vector<LineDim> lds, int dim,
   a.T = (int32_t)T;
   a.lds_w1_off = off;
   pp.lds_bytes = bytes;
-  // Lines whose FFT has a direct prime stage (radix 7 and up) or runs in the
-  // Bluestein form are arithmetic-heavy: twice the threads per tile hide
-  // more of it (measured 13-30 % faster on such passes; the power-of-two
-  // and 3/5-smooth passes measured 3-15 % slower that way)
+  // Lines whose FFT has a direct prime stage (radix 7 and up) are
+  // arithmetic-heavy: twice the threads per tile hide more of it (measured
+  // 13-30 % faster on such passes; the power-of-two and 3/5-smooth passes
+  // measured 3-15 % slower that way)
   bool direct_prime = false;
   for (int i = 0; i < a.nstages; ++i) direct_prime = direct_prime || (a.radix[i] > 5 && a.radix[i] != 8);
-  pp.threads = (a.bs_M || direct_prime) ? kBlockThreadsHeavy : kBlockThreads;
+  pp.threads = direct_prime ? kBlockThreadsHeavy : kBlockThreads;
   int64_t nt = (a.ldim[0] + T - 1) / T;
   for (int i = 1; i < a.D; ++i) nt *= a.ldim[i];
   a.ntiles = nt;
   pp.grid = std::min<int64_t>(nt, 1 << 20);
-  line_setup(p, pp);
-  a.scale = 1.0;
-  a.do_scale = 0;
-  pp.gen_args = a;
-  pp.gen_threads = pp.threads;
-  pp.gen_lds = pp.lds_bytes;
-  pp.gen_grid = pp.grid;
-  return PFFT_OK;
+  return keep_generic();
 }
 
 // Four-step form of a c2c line too long for one LDS-resident pass: M = M1 M2

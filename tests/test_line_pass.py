@@ -1,8 +1,8 @@
-"""The line pass (register-resident lines of any 13-smooth length) against the
-FP64 oracle, where it can go wrong: every radix by itself (lines of 2 to 16
-points, one stage, no LDS), two and three stages, odd r2c / c2r, tiles with
-fewer lines than they hold, both memory orders, extra dims, long lines with one
-or two lines to a tile.  On the CPU through the host emulator, which runs the
+"""The line pass against the FP64 oracle, where it can go wrong: every radix by
+itself (lines of 2 to 16 points, one stage, no LDS), two and three stages, odd
+r2c / c2r, tiles with fewer lines than they hold, both memory orders, extra
+dims, long lines with one or two lines to a tile, prime factors of 17 to 61 (one,
+two, a square), Bluestein lengths.  On the CPU through the host emulator, which runs the
 kernel's own phase functions; on the device with the specialised kernels off,
 so that every pass takes the line pass.  Tolerances (relative L2): Float64
 1e-13, Float32 5e-7 log2 N."""
@@ -18,12 +18,14 @@ SIZES = [(n, 5, 3) for n in range(2, 17)]            # one stage
 SIZES += [(n, 37, 2) for n in (26, 33, 45, 98, 121, 143, 144, 169, 196, 225, 256)]   # two
 SIZES += [(n, 19) for n in (315, 448, 1001, 2025, 4096)]   # three, and 4-stage 2 n of R2R
 SIZES += [(3, 2, 130), (2, 70, 9)]                   # short lines, many of them
+SIZES += [(n, 37, 2) for n in (17, 31, 34, 59, 61, 122, 289, 323)]   # primes 17 to 61
+SIZES += [(n, 5, 3) for n in (67, 134, 257)] + [(1031, 3)]    # Bluestein
 
 
 def cases_of(T, dims):
     yield "RFFT", (T.RFFT(),)
     yield "FFT", (T.FFT(),)
-    if dims[0] <= 256:
+    if dims[0] <= 323:
         for k in R2R_KINDS:
             yield k, (T.R2R(getattr(T, k)),)
 
