@@ -29,13 +29,14 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
 
 PRODUCT_SOURCES = ["kernels.hip", "fast.hip", "fast_nt.hip", "plan.cpp", "capi.cpp"]
 # line_kernel.hip holds one kernel per precision, form (direct, Bluestein, prime
-# factors of 17 to 61) and class: (object, defines)
+# factors of 17 to 61, small arrays) and class: (object, defines)
 LINE_CLASSES = 7
 LINE_OBJECTS = [("line_%s_%s%d.o" % (name, form, c),
                  ["-DPFFT_LINE_REAL=" + real, "-DPFFT_LINE_NAME=%s_%s" % (name, form),
                   "-DPFFT_LINE_FORM=%d" % k, "-DPFFT_LINE_CLASS=%d" % c])
-                for c in reversed(range(LINE_CLASSES)) for k, form in enumerate(("", "bs", "prime"))
-                for real, name in (("double", "f64"), ("float", "f32"))]
+                for c in reversed(range(LINE_CLASSES)) for k, form in enumerate(("", "bs", "prime", "small"))
+                for real, name in (("double", "f64"), ("float", "f32"))
+                if not (c == 5 and form in ("", "small"))]   # (R2R: no direct forms)
 EMU_SOURCES = ["emu.cpp", "plan.cpp"]
 
 

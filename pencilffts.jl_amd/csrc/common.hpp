@@ -148,8 +148,9 @@ struct LineStage {
 };
 
 // How the line FFT is done (line_pass.hpp, line_bluestein.hpp, line_prime.hpp)
-enum LineForm : int32_t { LF_DIRECT = 0, LF_BLUESTEIN = 1, LF_PRIME = 2 };
-constexpr int kLineForms = 3;
+// (LF_SMALL: the direct form with one butterfly a thread)
+enum LineForm : int32_t { LF_DIRECT = 0, LF_BLUESTEIN = 1, LF_PRIME = 2, LF_SMALL = 3 };
+constexpr int kLineForms = 4;
 // Largest workgroup: float R2R kinds in the Bluestein form may need 8192 points
 // for each of two lines (the parts of complex data).
 constexpr int line_max_threads(int cls, int form, bool f32) {
@@ -164,6 +165,9 @@ struct LineArgs {
   uint32_t pitch, sh;    // LDS line pitch (points); a pad slot after every 2^sh points
   uint32_t m_half, m_line;   // reciprocals of M / 2 + 1 and M
   int32_t jf_in, jf_out; // contiguous side: neighbouring threads along the line
+  uint32_t blocks;       // tiles along line dim 0
+  uint64_t m_blocks;     // its reciprocal, and those of line dims 1.. (line_div64)
+  uint64_t m_dim[kMaxDims];
   const void* tw;
   LineStage st[kLineStages];
 };

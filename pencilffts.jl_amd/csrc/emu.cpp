@@ -38,7 +38,7 @@ static void emu_pass(const PassPlan& pp, const PassArgs& a) {
 }
 
 // The line pass: every thread's registers live across the barriers.
-template <typename R, int CLS>
+template <typename R, int CLS, int PTS>
 static void emu_line(const PassPlan& pp, const PassArgs& a, const LineArgs& b) {
   const int nthr = (int)b.threads;
   std::vector<char> store((size_t)pp.lds_bytes + 16);
@@ -49,19 +49,18 @@ static void emu_line(const PassPlan& pp, const PassArgs& a, const LineArgs& b) {
   const LineOp<R> op(a);
   for (int64_t tile = 0; tile < a.ntiles; ++tile) {
     TileCtx c;
-    tile_init(a, tile, c);
-    int64_t m0;
-    const OpLine<R> o = a.op ? op_tile<R>(a, tile, &m0) : OpLine<R>{R(0), R(1)};
+    line_tile(a, b, (uint32_t)tile, c);
+    const OpLine<R> o = a.op ? op.tile(a, b, (uint32_t)tile) : OpLine<R>{R(0), R(1)};
     for (int s = 0; s < b.S; ++s) {
       const bool fin = s == b.S - 1;
       for (int t = 0; t < nthr; ++t) {
         cpx<R>* v = &regs[(size_t)t * kLinePoints];
         if (s == 0) {
-#define PFFT_F(RAD) line_first<R, CLS, RAD>(a, b, c, op, o, t, v)
+#define PFFT_F(RAD) line_first<R, CLS, PTS, RAD>(a, b, c, op, o, t, v)
           PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
 #undef PFFT_F
         } else {
-#define PFFT_F(RAD) line_get<R, RAD>(b, c, s, fin && direct && b.jf_out, t, v, W)
+#define PFFT_F(RAD) line_get<R, PTS, RAD>(b, c, s, fin && direct && b.jf_out, t, v, W)
           PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
 #undef PFFT_F
         }
@@ -69,11 +68,11 @@ static void emu_line(const PassPlan& pp, const PassArgs& a, const LineArgs& b) {
       for (int t = 0; t < nthr; ++t) {
         cpx<R>* v = &regs[(size_t)t * kLinePoints];
         if (fin && direct) {
-#define PFFT_F(RAD) line_store<R, CLS, RAD>(a, b, c, op, o, t, v)
+#define PFFT_F(RAD) line_store<R, CLS, PTS, RAD>(a, b, c, op, o, t, v)
           PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
 #undef PFFT_F
         } else {
-#define PFFT_F(RAD) line_put<R, RAD>(a, b, c, s, fin, t, v, W)
+#define PFFT_F(RAD) line_put<R, PTS, RAD>(a, b, c, s, s == 0 && b.jf_in, fin, t, v, W)
           PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
 #undef PFFT_F
         }
@@ -93,12 +92,11 @@ static void emu_line_bs(const PassPlan& pp, const PassArgs& a, const LineArgs& b
   const LineOp<R> op(a);
   for (int64_t tile = 0; tile < a.ntiles; ++tile) {
     TileCtx c;
-    tile_init(a, tile, c);
-    int64_t m0;
-    const OpLine<R> o = a.op ? op_tile<R>(a, tile, &m0) : OpLine<R>{R(0), R(1)};
+    line_tile(a, b, (uint32_t)tile, c);
+    const OpLine<R> o = a.op ? op.tile(a, b, (uint32_t)tile) : OpLine<R>{R(0), R(1)};
     for (int t = 0; t < nthr; ++t) {
 #define PFFT_F(RAD) bs_first<R, CLS, RAD>(a, b, c, op, o, t, W)
-      PFFT_LINE_RADIX(b.st[0].rad, PFFT_F)
+      PFFT_LINE_RADIX_POW2(b.st[0].rad, PFFT_F)
 #undef PFFT_F
     }
     for (int i = 1; i < 2 * b.S - 2; ++i) {
@@ -106,13 +104,13 @@ static void emu_line_bs(const PassPlan& pp, const PassArgs& a, const LineArgs& b
       const int dir = i < b.S - 1 ? 0 : i == b.S - 1 ? 1 : 2;
       for (int t = 0; t < nthr; ++t) {
 #define PFFT_F(RAD) bs_stage<R, RAD>(a, b, c, s, dir, t, W)
-        PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
+        PFFT_LINE_RADIX_POW2(b.st[s].rad, PFFT_F)
 #undef PFFT_F
       }
     }
     for (int t = 0; t < nthr; ++t) {
 #define PFFT_F(RAD) bs_last<R, CLS, RAD>(a, b, c, op, o, t, W)
-      PFFT_LINE_RADIX(b.st[0].rad, PFFT_F)
+      PFFT_LINE_RADIX_POW2(b.st[0].rad, PFFT_F)
 #undef PFFT_F
     }
     if (!line_direct(CLS))
@@ -131,9 +129,8 @@ static void emu_line_prime(const PassPlan& pp, const PassArgs& a, const LineArgs
   const LineOp<R> op(a);
   for (int64_t tile = 0; tile < a.ntiles; ++tile) {
     TileCtx c;
-    tile_init(a, tile, c);
-    int64_t m0;
-    const OpLine<R> o = a.op ? op_tile<R>(a, tile, &m0) : OpLine<R>{R(0), R(1)};
+    line_tile(a, b, (uint32_t)tile, c);
+    const OpLine<R> o = a.op ? op.tile(a, b, (uint32_t)tile) : OpLine<R>{R(0), R(1)};
     for (int t = 0; t < nthr; ++t) prime_load<R, CLS>(a, b, c, op, o, t, W);
     for (int s = 0; s < b.S; ++s) {
       const bool fin = s == b.S - 1;
@@ -144,13 +141,13 @@ static void emu_line_prime(const PassPlan& pp, const PassArgs& a, const LineArgs
       }
       for (int t = 0; t < nthr; ++t) {
         cpx<R>* v = &regs[(size_t)t * kLinePoints];
-#define PFFT_F(RAD) line_get<R, RAD>(b, c, s, false, t, v, W)
+#define PFFT_F(RAD) line_get<R, kLinePoints, RAD>(b, c, s, false, t, v, W)
         PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
 #undef PFFT_F
       }
       for (int t = 0; t < nthr; ++t) {
         cpx<R>* v = &regs[(size_t)t * kLinePoints];
-#define PFFT_F(RAD) line_put<R, RAD>(a, b, c, s, fin, t, v, W)
+#define PFFT_F(RAD) line_put<R, kLinePoints, RAD>(a, b, c, s, false, fin, t, v, W)
         PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
 #undef PFFT_F
       }
@@ -166,7 +163,10 @@ template <typename R, int CLS>
 static void emu_form(const PassPlan& pp, const PassArgs& a, const LineArgs& b) {
   if (b.form == LF_BLUESTEIN) emu_line_bs<R, CLS>(pp, a, b);
   else if (b.form == LF_PRIME) emu_line_prime<R, CLS>(pp, a, b);
-  else emu_line<R, CLS>(pp, a, b);
+  else if constexpr (CLS != LC_R2R) {
+    if (b.form == LF_SMALL) emu_line<R, CLS, 1>(pp, a, b);
+    else emu_line<R, CLS, kLinePoints>(pp, a, b);
+  }
 }
 
 template <typename R>

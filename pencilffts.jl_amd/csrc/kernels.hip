@@ -78,14 +78,17 @@ static void launch_generic_t(const PassPlan& pp, const PassArgs& a, hipStream_t 
 }
 // ---- line pass ------------------------------------------------------------------
 // its kernels, one object per precision, form and class (line_kernel.hip)
-#define PFFT_LINE_SET(X, t) X(t, 0) X(t, 1) X(t, 2) X(t, 3) X(t, 4) X(t, 5) X(t, 6)
-#define PFFT_LINE_EACH(X)                                                          \
-  PFFT_LINE_SET(X, f32_) PFFT_LINE_SET(X, f32_bs) PFFT_LINE_SET(X, f32_prime)     \
-  PFFT_LINE_SET(X, f64_) PFFT_LINE_SET(X, f64_bs) PFFT_LINE_SET(X, f64_prime)
+// (the R2R class, 5, has no direct forms)
+#define PFFT_LINE_SET(X, t) X(t, 0) X(t, 1) X(t, 2) X(t, 3) X(t, 4)
+#define PFFT_LINE_ALL(X, t) PFFT_LINE_SET(X, t) X(t, 5) X(t, 6)
+#define PFFT_LINE_PAIR(X, t) PFFT_LINE_SET(X, t) X(t, 6)
 #define PFFT_X(t, c)                              \
   int line_prepare_##t##c(const PassPlan& pp);    \
   void line_launch_##t##c(const PassPlan& pp, const PassArgs& a, const LineArgs& b, hipStream_t st);
-PFFT_LINE_EACH(PFFT_X)
+PFFT_LINE_PAIR(PFFT_X, f32_) PFFT_LINE_PAIR(PFFT_X, f32_small)
+PFFT_LINE_ALL(PFFT_X, f32_bs) PFFT_LINE_ALL(PFFT_X, f32_prime)
+PFFT_LINE_PAIR(PFFT_X, f64_) PFFT_LINE_PAIR(PFFT_X, f64_small)
+PFFT_LINE_ALL(PFFT_X, f64_bs) PFFT_LINE_ALL(PFFT_X, f64_prime)
 #undef PFFT_X
 struct LineKernel {
   int (*prepare)(const PassPlan&);
@@ -93,7 +96,13 @@ struct LineKernel {
 };
 static const LineKernel& line_kernel(int real_type, int form, int cls) {
 #define PFFT_X(t, c) {line_prepare_##t##c, line_launch_##t##c},
-  static const LineKernel k[2 * kLineForms * kLineClasses] = {PFFT_LINE_EACH(PFFT_X)};
+#define PFFT_HALF(t) PFFT_LINE_SET(PFFT_X, t) {nullptr, nullptr}, PFFT_X(t, 6)
+  static const LineKernel k[2 * kLineForms * kLineClasses] = {   // in LineForm order
+      PFFT_HALF(f32_) PFFT_LINE_ALL(PFFT_X, f32_bs) PFFT_LINE_ALL(PFFT_X, f32_prime)
+      PFFT_HALF(f32_small)
+      PFFT_HALF(f64_) PFFT_LINE_ALL(PFFT_X, f64_bs) PFFT_LINE_ALL(PFFT_X, f64_prime)
+      PFFT_HALF(f64_small)};
+#undef PFFT_HALF
 #undef PFFT_X
   return k[((real_type == PFFT_F32 ? 0 : kLineForms) + form) * kLineClasses + cls];
 }

@@ -23,25 +23,41 @@ __device__ __forceinline__ uint32_t opaque(uint32_t x) {
   return x;
 }
 
+// Touches every cache line of the kernel's arguments at once.  Read where they
+// are first needed they miss one after the other, each miss a trip to the
+// memory the host wrote them to: the first global load of a pass then left
+// 1.8 us after the wavefront started, half the time of a pass on a small array
+// (0.9 us with this, the reciprocals of line_tile and opaque_s).
+__device__ __forceinline__ void touch_args() {
+  static_assert(sizeof(PassArgs) + sizeof(LineArgs) > 15 * 64 &&
+                    sizeof(PassArgs) + sizeof(LineArgs) <= 16 * 64,
+                "one word of each 64 bytes");
+  const auto* k = (const __attribute__((address_space(4))) uint32_t*)
+      __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" ::"s"(k[0]), "s"(k[16]), "s"(k[32]), "s"(k[48]), "s"(k[64]), "s"(k[80]),
+               "s"(k[96]), "s"(k[112]), "s"(k[128]), "s"(k[144]), "s"(k[160]), "s"(k[176]),
+               "s"(k[192]), "s"(k[208]), "s"(k[224]), "s"(k[240]));
+}
+
 #if PFFT_LINE_FORM == 1
 // (float: held to 128 VGPRs, 4 waves per SIMD; it asks for 130)
 template <typename R, int CLS>
 __global__ __launch_bounds__(line_max_threads(CLS, LF_BLUESTEIN, sizeof(R) == 4),
                              sizeof(R) == 4 ? 4 : 2) void k_line_bs(PassArgs a, LineArgs b) {
+  touch_args();
   extern __shared__ __align__(16) char lds[];
   cpx<R>* W = (cpx<R>*)lds;
   const uint32_t tid = threadIdx.x;
   const LineOp<R> op(a);
   for (int64_t tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x) {
     TileCtx c;
-    tile_init(a, tile, c);
+    line_tile(a, b, (uint32_t)tile, c);
     OpLine<R> o = {R(0), R(1)};
     if constexpr (CLS == LC_C2C_OP) {
-      int64_t m0;
-      if (op.op) o = op_tile<R>(a, tile, &m0);
+      if (op.op) o = op.tile(a, b, (uint32_t)tile);
     }
 #define PFFT_F(RAD) bs_first<R, CLS, RAD>(a, b, c, op, o, opaque(tid), W)
-    PFFT_LINE_RADIX(b.st[0].rad, PFFT_F)
+    PFFT_LINE_RADIX_POW2(b.st[0].rad, PFFT_F)
 #undef PFFT_F
     __syncthreads();
     // forward stages 1 .. S-2, the middle one, backward S-2 .. 1
@@ -49,12 +65,12 @@ __global__ __launch_bounds__(line_max_threads(CLS, LF_BLUESTEIN, sizeof(R) == 4)
       const int s = i < b.S ? i : 2 * b.S - 2 - i;
       const int dir = i < b.S - 1 ? 0 : i == b.S - 1 ? 1 : 2;
 #define PFFT_F(RAD) bs_stage<R, RAD>(a, b, c, s, dir, opaque(tid), W)
-      PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
+      PFFT_LINE_RADIX_POW2(b.st[s].rad, PFFT_F)
 #undef PFFT_F
       __syncthreads();
     }
 #define PFFT_F(RAD) bs_last<R, CLS, RAD>(a, b, c, op, o, opaque(tid), W)
-    PFFT_LINE_RADIX(b.st[0].rad, PFFT_F)
+    PFFT_LINE_RADIX_POW2(b.st[0].rad, PFFT_F)
 #undef PFFT_F
     if constexpr (!line_direct(CLS)) {
       __syncthreads();
@@ -63,21 +79,21 @@ __global__ __launch_bounds__(line_max_threads(CLS, LF_BLUESTEIN, sizeof(R) == 4)
     __syncthreads();
   }
 }
-#define PFFT_LINE_KERNEL k_line_bs
+#define PFFT_LINE_KERNEL k_line_bs<PFFT_LINE_REAL, PFFT_LINE_CLASS>
 #elif PFFT_LINE_FORM == 2
 template <typename R, int CLS>
 __global__ __launch_bounds__(kLineMaxThreads) void k_line_prime(PassArgs a, LineArgs b) {
+  touch_args();
   extern __shared__ __align__(16) char lds[];
   cpx<R>* W = (cpx<R>*)lds;
   const uint32_t tid = threadIdx.x;
   const LineOp<R> op(a);
   for (int64_t tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x) {
     TileCtx c;
-    tile_init(a, tile, c);
+    line_tile(a, b, (uint32_t)tile, c);
     OpLine<R> o = {R(0), R(1)};
     if constexpr (CLS == LC_C2C_OP) {
-      int64_t m0;
-      if (op.op) o = op_tile<R>(a, tile, &m0);
+      if (op.op) o = op.tile(a, b, (uint32_t)tile);
     }
     prime_load<R, CLS>(a, b, c, op, o, tid, W);
     __syncthreads();
@@ -89,12 +105,11 @@ __global__ __launch_bounds__(kLineMaxThreads) void k_line_prime(PassArgs a, Line
         __syncthreads();
         prime_put<R>(a, b, c, s, fin, tid, v, W);
       } else {
-        // (a prime came first: s > 0)
         cpx<R> v[kLinePoints];
 #define PFFT_F(RAD)                                       \
-  line_get<R, RAD>(b, c, s, false, opaque(tid), v, W);    \
+  line_get<R, kLinePoints, RAD>(b, c, s, false, opaque(tid), v, W);    \
   __syncthreads();                                        \
-  line_put<R, RAD>(a, b, c, s, fin, opaque(tid), v, W)
+  line_put<R, kLinePoints, RAD>(a, b, c, s, false, fin, opaque(tid), v, W)
         PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
 #undef PFFT_F
       }
@@ -105,10 +120,11 @@ __global__ __launch_bounds__(kLineMaxThreads) void k_line_prime(PassArgs a, Line
     __syncthreads();
   }
 }
-#define PFFT_LINE_KERNEL k_line_prime
+#define PFFT_LINE_KERNEL k_line_prime<PFFT_LINE_REAL, PFFT_LINE_CLASS>
 #else
-template <typename R, int CLS>
+template <typename R, int CLS, int PTS>
 __global__ __launch_bounds__(kLineMaxThreads) void k_line(PassArgs a, LineArgs b) {
+  touch_args();
   extern __shared__ __align__(16) char lds[];
   cpx<R>* W = (cpx<R>*)lds;
   const uint32_t tid = threadIdx.x;
@@ -116,31 +132,30 @@ __global__ __launch_bounds__(kLineMaxThreads) void k_line(PassArgs a, LineArgs b
   const LineOp<R> op(a);
   for (int64_t tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x) {
     TileCtx c;
-    tile_init(a, tile, c);
+    line_tile(a, b, (uint32_t)tile, c);
     OpLine<R> o = {R(0), R(1)};
     if constexpr (CLS == LC_C2C_OP) {
-      int64_t m0;
-      if (op.op) o = op_tile<R>(a, tile, &m0);
+      if (op.op) o = op.tile(a, b, (uint32_t)tile);
     }
     cpx<R> v[kLinePoints];
     // stage s leaves its butterflies in LDS, or (fin, direct) in memory
     const bool one = b.S == 1;
 #define PFFT_F(RAD)                                                          \
-  line_first<R, CLS, RAD>(a, b, c, op, o, opaque(tid), v);                     \
-  if (direct && one) line_store<R, CLS, RAD>(a, b, c, op, o, opaque(tid), v);  \
-  else line_put<R, RAD>(a, b, c, 0, one, opaque(tid), v, W)
+  line_first<R, CLS, PTS, RAD>(a, b, c, op, o, opaque(tid), v);                     \
+  if (direct && one) line_store<R, CLS, PTS, RAD>(a, b, c, op, o, opaque(tid), v);  \
+  else line_put<R, PTS, RAD>(a, b, c, 0, b.jf_in, one, opaque(tid), v, W)
     PFFT_LINE_RADIX(b.st[0].rad, PFFT_F)
 #undef PFFT_F
     for (int s = 1; s < b.S; ++s) {
       const bool fin = s == b.S - 1;
       __syncthreads();
 #define PFFT_F(RAD)                                                          \
-  line_get<R, RAD>(b, c, s, direct && fin && b.jf_out, opaque(tid), v, W);   \
+  line_get<R, PTS, RAD>(b, c, s, direct && fin && b.jf_out, opaque(tid), v, W);   \
   if (direct && fin) {                                                       \
-    line_store<R, CLS, RAD>(a, b, c, op, o, opaque(tid), v);                 \
+    line_store<R, CLS, PTS, RAD>(a, b, c, op, o, opaque(tid), v);                 \
   } else {                                                                   \
     __syncthreads();                                                         \
-    line_put<R, RAD>(a, b, c, s, fin, opaque(tid), v, W);                    \
+    line_put<R, PTS, RAD>(a, b, c, s, false, fin, opaque(tid), v, W);                    \
   }
       PFFT_LINE_RADIX(b.st[s].rad, PFFT_F)
 #undef PFFT_F
@@ -153,13 +168,14 @@ __global__ __launch_bounds__(kLineMaxThreads) void k_line(PassArgs a, LineArgs b
   }
 }
 
-#define PFFT_LINE_KERNEL k_line
+#define PFFT_LINE_KERNEL \
+  k_line<PFFT_LINE_REAL, PFFT_LINE_CLASS, PFFT_LINE_FORM == LF_SMALL ? 1 : kLinePoints>
 #endif
 
 int PFFT_CAT3(line_prepare_, PFFT_LINE_NAME, PFFT_LINE_CLASS)(const PassPlan& pp) {
   if (pp.lds_bytes <= 64 * 1024) return PFFT_OK;
   const hipError_t e =
-      hipFuncSetAttribute((const void*)PFFT_LINE_KERNEL<PFFT_LINE_REAL, PFFT_LINE_CLASS>,
+      hipFuncSetAttribute((const void*)PFFT_LINE_KERNEL,
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)pp.lds_bytes);
   if (e != hipSuccess)
     return fail(PFFT_ERR_DEVICE, std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
@@ -169,7 +185,7 @@ int PFFT_CAT3(line_prepare_, PFFT_LINE_NAME, PFFT_LINE_CLASS)(const PassPlan& pp
 void PFFT_CAT3(line_launch_, PFFT_LINE_NAME, PFFT_LINE_CLASS)(const PassPlan& pp,
                                                               const PassArgs& a,
                                                               const LineArgs& b, hipStream_t st) {
-  hipLaunchKernelGGL((PFFT_LINE_KERNEL<PFFT_LINE_REAL, PFFT_LINE_CLASS>),
+  hipLaunchKernelGGL((PFFT_LINE_KERNEL),
                      dim3((unsigned)pp.grid), dim3(b.threads), (size_t)pp.lds_bytes, st, a, b);
 }
 

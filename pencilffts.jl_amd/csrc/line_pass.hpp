@@ -1,14 +1,14 @@
 // Line pass: lines of any length whose FFT length factors into radices of 2
-// to 16, any transform kind and any layout, float or double.
+// to 16, complex FFTs, r2c and c2r in any layout, float or double.  (The R2R
+// kinds and lengths with larger primes: line_prime.hpp, line_bluestein.hpp.)
 //
 // One workgroup transforms a tile of lines.  Every thread holds 16 points of
 // the tile in registers (one radix-9..16 butterfly, two of radix 6..8, ...):
-//   first   global memory -> registers (with the kind's input reorder,
-//           merge or twiddle), first butterflies, registers -> LDS
+//   first   global memory -> registers (with the c2r's merge), first
+//           butterflies, registers -> LDS
 //   middle  LDS -> registers, twiddles, butterflies, back to the same LDS lines
-//   last    LDS -> registers, twiddles, butterflies; complex FFTs and c2r store
-//           from the registers, the other kinds put the transform into LDS
-//           and run their post-processing from there
+//   last    LDS -> registers, twiddles, butterflies, stored from the registers
+//           (the even r2c puts the transform into LDS and splits it from there)
 // A stage moves points within the line, so a barrier lies between its reads
 // and its writes: one LDS copy of the tile, S - 1 trips through it for S
 // radices, S <= 3 up to 4096 points.
@@ -38,8 +38,18 @@
 
 namespace pfft {
 
-// butterflies of one radix a thread holds
-constexpr int line_bpt(int rad) { return kLinePoints / rad; }
+// butterflies of one radix a thread holds: as many as fit pts points
+constexpr int line_bpt(int rad, int pts = kLinePoints) { return pts / rad > 1 ? pts / rad : 1; }
+
+// A copy of the uniform value x the compiler knows nothing about: the products
+// of a step with every r of every radix stay in their case instead of filling
+// the launch's first instructions (and spilling there).
+PFFT_HD uint64_t opaque_s(uint64_t x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+s"(x));
+#endif
+  return x;
+}
 
 // x / d for the divisors of the index maps (m = ceil(2^32 / d), 0 for d = 1;
 // exact while x d < 2^32)
@@ -57,6 +67,39 @@ template <typename R>
 PFFT_HD void lds_put(cpx<R>* p, cpx<R> z) {
   typedef R v2 __attribute__((ext_vector_type(2)));
   *(v2*)p = v2{z.re, z.im};
+}
+
+// x / d for tile indexes (below 2^31): m = ceil(2^64 / d), 0 for d = 1
+PFFT_HD uint32_t line_div64(uint32_t x, uint64_t m) {
+  if (!m) return x;
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (uint32_t)__umul64hi((uint64_t)x, m);
+#else
+  return (uint32_t)(((unsigned __int128)x * m) >> 64);
+#endif
+}
+
+// tile_init by reciprocals (tiles always in ascending order, line dim 0 first)
+PFFT_HD void line_tile(const PassArgs& a, const LineArgs& b, uint32_t tile, TileCtx& c) {
+  uint32_t rest = line_div64(tile, b.m_blocks);
+  const uint32_t b0 = tile - rest * b.blocks;
+  const int64_t m0 = (int64_t)b0 * a.T;
+  int64_t ib = m0 * a.lsin[0], ob = m0 * a.lsout[0];
+  for (int d = 1; d < a.D; ++d) {
+    const uint32_t q = d + 1 < a.D ? line_div64(rest, b.m_dim[d]) : 0;
+    const int64_t m = rest - q * (uint32_t)a.ldim[d];
+    rest = q;
+    ib += m * a.lsin[d];
+    ob += m * a.lsout[d];
+  }
+  c.in_base = ib;
+  c.out_base = ob;
+  const int64_t left = a.ldim[0] - m0;
+  c.Tact = (int32_t)(left < a.T ? left : a.T);
+  c.tile = tile;
+  c.m0 = m0;
+  const int32_t nreal = a.r2r_cplx ? 2 * c.Tact : c.Tact;
+  c.Tw = a.pair_real ? (nreal + 1) / 2 : nreal;
 }
 
 // Thread tid's i-th butterfly of a stage: line w and index j; jf: the
@@ -186,6 +229,17 @@ struct LineOp {
     else o.a += k * k;
     return o;
   }
+  // the part of a tile: its line dims 1 .. D - 1 (as op_tile)
+  PFFT_HD OpLine<R> tile(const PassArgs& a, const LineArgs& b, uint32_t t) const {
+    OpLine<R> o = {R(0), R(1)};
+    uint32_t rest = line_div64(t, b.m_blocks);
+    for (int d = 1; d < a.D; ++d) {
+      const uint32_t q = d + 1 < a.D ? line_div64(rest, b.m_dim[d]) : 0;
+      op_add<R>(a, d, (int)(rest - q * (uint32_t)a.ldim[d]), o);
+      rest = q;
+    }
+    return o;
+  }
   // points j + r nb of one line times alpha m(k)
   template <int RAD>
   PFFT_HD void apply(const OpLine<R>& o, uint32_t j, uint32_t nb, cpx<R>* x) const {
@@ -208,10 +262,10 @@ struct LineOp {
 
 // ---- first stage: global memory -> butterflies ----------------------------------
 // op, otile: the operator and its part shared by the tile (LC_C2C_OP)
-template <typename R, int CLS, int RAD>
+template <typename R, int CLS, int PTS, int RAD>
 PFFT_HD void line_first(const PassArgs& a, const LineArgs& b, const TileCtx& c,
                         const LineOp<R>& op, const OpLine<R>& otile, uint32_t tid, cpx<R>* v) {
-  constexpr int BPT = line_bpt(RAD);
+  constexpr int BPT = line_bpt(RAD, PTS);
   const LineStage& st = b.st[0];
   const uint32_t ls = (uint32_t)a.lsin[0], sk = (uint32_t)a.sk_in;
   const bool jf = b.jf_in != 0;
@@ -220,7 +274,7 @@ PFFT_HD void line_first(const PassArgs& a, const LineArgs& b, const TileCtx& c,
   // below 2^31 bytes).
   constexpr uint32_t esz = sizeof(R) * (CLS == LC_R2C || CLS == LC_R2C_ODD ? 1 : 2);
   const char* base = (const char*)a.in + c.in_base * (int64_t)esz;
-  const uint64_t step = (uint64_t)st.nb * a.sk_in * esz * (CLS == LC_R2C ? 2 : 1);
+  const uint64_t step = opaque_s((uint64_t)st.nb * a.sk_in * esz * (CLS == LC_R2C ? 2 : 1));
 #pragma unroll
   for (int i = 0; i < BPT; ++i) {
     uint32_t w, j;
@@ -283,8 +337,7 @@ PFFT_HD void line_first(const PassArgs& a, const LineArgs& b, const TileCtx& c,
         x[r] = up ? conj(z) : z;
       }
     } else {
-#pragma unroll
-      for (int r = 0; r < RAD; ++r) x[r] = line_point<R>(a, c, w, j + r * st.nb);
+      static_assert(CLS != CLS, "the R2R kinds load through LDS (line_prime.hpp)");
     }
     if (cj) {
 #pragma unroll
@@ -297,14 +350,13 @@ PFFT_HD void line_first(const PassArgs& a, const LineArgs& b, const TileCtx& c,
 
 // ---- LDS slots ------------------------------------------------------------------
 // Registers -> LDS after stage s: butterfly j = jq Ns + jj leaves point
-// jq Ns RAD + jj + r Ns in register r.  fin: the last stage, with a backward
-// transform's outer conjugation.
-template <typename R, int RAD>
-PFFT_HD void line_put(const PassArgs& a, const LineArgs& b, const TileCtx& c, int s, bool fin,
-                      uint32_t tid, const cpx<R>* v, cpx<R>* W) {
-  constexpr int BPT = line_bpt(RAD);
+// jq Ns RAD + jj + r Ns in register r; jf: as the butterflies were read.  fin:
+// the last stage, with a backward transform's outer conjugation.
+template <typename R, int PTS, int RAD>
+PFFT_HD void line_put(const PassArgs& a, const LineArgs& b, const TileCtx& c, int s, bool jf,
+                      bool fin, uint32_t tid, const cpx<R>* v, cpx<R>* W) {
+  constexpr int BPT = line_bpt(RAD, PTS);
   const LineStage& st = b.st[s];
-  const bool jf = s == 0 && b.jf_in;
   const bool cj = fin && a.bwd;
 #pragma unroll
   for (int i = 0; i < BPT; ++i) {
@@ -321,13 +373,13 @@ PFFT_HD void line_put(const PassArgs& a, const LineArgs& b, const TileCtx& c, in
   }
 }
 
-// LDS -> registers, twiddles, butterflies of stage s >= 1: point j + r nb of
-// the line times w_(Ns RAD)^(r jj); jf: the last stage before a contiguous
+// LDS -> registers, twiddles, butterflies of stage s: point j + r nb of the
+// line times w_(Ns RAD)^(r jj) (none in stage 0 of the lines loaded into LDS); jf: the last stage before a contiguous
 // store.
-template <typename R, int RAD>
+template <typename R, int PTS, int RAD>
 PFFT_HD void line_get(const LineArgs& b, const TileCtx& c, int s, bool jf, uint32_t tid, cpx<R>* v,
                       const cpx<R>* W) {
-  constexpr int BPT = line_bpt(RAD);
+  constexpr int BPT = line_bpt(RAD, PTS);
   const LineStage& st = b.st[s];
   const cpx<R>* tw = (const cpx<R>*)b.tw + st.tw;
 #pragma unroll
@@ -338,8 +390,10 @@ PFFT_HD void line_get(const LineArgs& b, const TileCtx& c, int s, bool jf, uint3
     const cpx<R>* L = W + w * b.pitch;
 #pragma unroll
     for (int r = 0; r < RAD; ++r) v[i * RAD + r] = lds_get(&L[wp(j + r * st.nb, b.sh)]);
+    if (s > 0) {
 #pragma unroll
-    for (int r = 1; r < RAD; ++r) v[i * RAD + r] = v[i * RAD + r] * tw[(r - 1) * st.ns + jj];
+      for (int r = 1; r < RAD; ++r) v[i * RAD + r] = v[i * RAD + r] * tw[(r - 1) * st.ns + jj];
+    }
   }
 #pragma unroll
   for (int i = 0; i < BPT; ++i) dft<R, RAD>(v + i * RAD);
@@ -347,18 +401,18 @@ PFFT_HD void line_get(const LineArgs& b, const TileCtx& c, int s, bool jf, uint3
 
 // ---- stores from the registers of the last stage ---------------------------------
 // Register r of butterfly j holds point j + r nb.
-template <typename R, int CLS, int RAD>
+template <typename R, int CLS, int PTS, int RAD>
 PFFT_HD void line_store(const PassArgs& a, const LineArgs& b, const TileCtx& c,
                         const LineOp<R>& op, const OpLine<R>& otile, uint32_t tid,
                         const cpx<R>* v) {
-  constexpr int BPT = line_bpt(RAD);
+  constexpr int BPT = line_bpt(RAD, PTS);
   const LineStage& st = b.st[b.S - 1];
   const uint32_t ls = (uint32_t)a.lsout[0], sk = (uint32_t)a.sk_out;
   const R sc = a.do_scale ? (R)a.scale : R(1);
   const R sci = a.bwd ? -sc : sc;
   constexpr uint32_t esz = sizeof(R) * (CLS == LC_C2R || CLS == LC_C2R_ODD ? 1 : 2);
   char* base = (char*)a.out + c.out_base * (int64_t)esz;
-  const uint64_t step = (uint64_t)st.nb * a.sk_out * esz * (CLS == LC_C2R ? 2 : 1);
+  const uint64_t step = opaque_s((uint64_t)st.nb * a.sk_out * esz * (CLS == LC_C2R ? 2 : 1));
 #pragma unroll
   for (int i = 0; i < BPT; ++i) {
     uint32_t w, j;
@@ -462,7 +516,14 @@ PFFT_HD void line_post(const PassArgs& a, const LineArgs& b, const TileCtx& c, u
 // direct: the last stage's registers hold the output
 constexpr bool line_direct(int cls) { return cls != LC_R2C && cls != LC_R2R; }
 
-// F<radix> for a run-time radix
+// F<radix> for a run-time radix; _POW2: for the powers of two
+#define PFFT_LINE_RADIX_POW2(rad, F) \
+  switch (rad) {                     \
+    case 2: F(2); break;             \
+    case 4: F(4); break;             \
+    case 8: F(8); break;             \
+    default: F(16); break;           \
+  }
 #define PFFT_LINE_RADIX(rad, F) \
   switch (rad) {                \
     case 2: F(2); break;        \

@@ -1,4 +1,5 @@
-// Line pass for FFT lengths with prime factors of 17 to 61.
+// Line pass for FFT lengths with prime factors of 17 to 61, and for the R2R kinds
+// of all lengths without larger ones.
 //
 // The tile is loaded into LDS, every radix is one trip through it, and the
 // outputs are stored from it.  A prime p takes its stage in the symmetric form
@@ -16,6 +17,9 @@
 // FFTs) measured slower and less exact at these factors: 306 x 170 x 190
 // complex floats 1254 us a pair against 1106 us in the generic phases, its
 // largest error 2.2e-6 against 1.2e-6.
+// The R2R kinds take this form for its load loop: their gathers, expanded for
+// every point of every radix's first butterfly, made kernels that took ten
+// minutes to compile, for one trip through LDS less.
 #pragma once
 
 #include "line_bluestein.hpp"

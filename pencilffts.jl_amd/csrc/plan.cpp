@@ -430,6 +430,8 @@ static void chain_perm(int N, int n, bool permute, int32_t* perm) {
 // ---- line pass (line_pass.hpp) ------------------------------------------------
 static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+constexpr int64_t kLineSmallThreads = 128 * 1024;
+
 // Threads per line of a schedule: the stage with the most butterflies per
 // thread slot decides.
 static double line_load(int64_t M, const int32_t* rad, int ns) {
@@ -438,13 +440,20 @@ static double line_load(int64_t M, const int32_t* rad, int ns) {
     worst = std::max(worst, (double)(M / rad[s]) / (kLinePoints / rad[s]));
   return worst;
 }
+// Points a thread goes through in all stages, a stage's barrier and index
+// arithmetic counted as ten more: what a launch of few wavefronts takes.
+static double line_depth(const int32_t* rad, int ns) {
+  double d = 10 * ns;
+  for (int s = 0; s < ns; ++s) d += rad[s];
+  return d;
+}
 
 // Radices of an M-point line: its prime factors of 17 to 61 first, then radices
 // of 2 to 16, descending: the fewest stages (each one more is another trip of
 // the line through LDS), then the fewest threads per line (a stage with fewer
-// points per thread than the others leaves threads idle).  0 where M does not
-// factor that way.
-static int line_schedule(int64_t M, int32_t* best) {
+// points per thread than the others leaves threads idle); small: the shortest
+// line_depth.  0 where M does not factor that way.
+static int line_schedule(int64_t M, int32_t* best, bool small = false) {
   int primes = 0;
   int64_t rest = M;
   for (int32_t q : {61, 59, 53, 47, 43, 41, 37, 31, 29, 23, 19, 17})
@@ -459,15 +468,15 @@ static int line_schedule(int64_t M, int32_t* best) {
   int32_t cur[kLineStages];
   auto rec = [&](auto&& self, int64_t m, int32_t top, int ns) -> void {
     if (m == 1) {
-      const double l = line_load(M, cur, ns);
-      if (!n_best || ns < n_best || (ns == n_best && l < load)) {
+      const double l = small ? line_depth(cur, ns) : line_load(M, cur, ns);
+      if (!n_best || (!small && ns < n_best) || ((small || ns == n_best) && l < load)) {
         n_best = ns;
         load = l;
         std::copy(cur, cur + ns, best + primes);
       }
       return;
     }
-    if (primes + ns == kLineStages || (n_best && ns >= n_best)) return;
+    if (primes + ns == kLineStages || (n_best && !small && ns >= n_best)) return;
     for (int32_t r = top; r >= 2; --r)
       if (m % r == 0) {
         cur[ns] = r;
@@ -602,11 +611,11 @@ static bool line_setup(Plan& p, PassPlan& pp) {
   if (a.kind == L_COPY || a.M < 2) return false;
   const int64_t M = a.bs_M ? a.bs_M : a.M;   // points per work line
   int32_t rad[kLineStages];
-  const int S = line_schedule(M, rad);
+  int S = line_schedule(M, rad);
   if (!S) return false;
-  b.S = S;
+  int64_t pts = kLinePoints;   // points a thread holds
   b.cls = line_class(a.kind);
-  b.form = a.bs_M ? LF_BLUESTEIN : rad[0] > 16 ? LF_PRIME : LF_DIRECT;
+  b.form = a.bs_M ? LF_BLUESTEIN : rad[0] > 16 || b.cls == LC_R2R ? LF_PRIME : LF_DIRECT;
   const int64_t max_threads = line_max_threads(b.cls, b.form, p.real_type == PFFT_F32);
   const int64_t rs = p.real_type == PFFT_F32 ? 4 : 8, cs = 2 * rs;
   const bool direct = b.cls != LC_R2C && b.cls != LC_R2R;
@@ -634,16 +643,16 @@ static bool line_setup(Plan& p, PassPlan& pp) {
     for (int s = 0; s < S; ++s) {
       const int64_t n = Tw * (M / rad[s]);   // butterflies
       t = std::max(t, rad[s] > 16 ? ceil_div(n, 64) * 64 * ceil_div((rad[s] - 1) / 2, kPrimePairs)
-                                  : ceil_div(n, kLinePoints / rad[s]));
+                                  : ceil_div(n, std::max<int64_t>(pts / rad[s], 1)));
     }
     return ceil_div(t, 64) * 64;
   };
   auto bytes = [&](int64_t Tw) {
-    return S == 1 && direct && b.form == LF_DIRECT ? 0 : Tw * pitch(Tw) * cs;
+    return S == 1 && direct && (b.form == LF_DIRECT || b.form == LF_SMALL) ? 0 : Tw * pitch(Tw) * cs;
   };
   // lane offsets: 32 bits within a tile
   auto reach = [&](int64_t T) -> int64_t {
-    if (b.form != LF_DIRECT) return 0;
+    if (b.form == LF_BLUESTEIN || b.form == LF_PRIME) return 0;
     const int64_t nb = M / rad[0], nbo = M / rad[S - 1];
     const int64_t ein = a.in_cplx ? cs : rs, eout = a.out_cplx ? cs : rs;
     const int64_t pin = b.cls == LC_R2C ? 2 : b.cls == LC_C2R_ODD ? rad[0] : 1;
@@ -651,7 +660,8 @@ static bool line_setup(Plan& p, PassPlan& pp) {
     return std::max(((T - 1) * a.lsin[0] + pin * nb * a.sk_in) * ein,
                     ((T - 1) * a.lsout[0] + pout * nbo * a.sk_out) * eout);
   };
-  // Tile: 128-byte runs on a transposed side and about 256 threads; fewer
+  // Tile: 128-byte runs on a transposed side and about 256 threads, more where
+  // they cost no threads (a prime stage works in whole wavefronts); fewer
   // lines where threads or LDS run out (two workgroups per CU at least), where
   // the grid would not fill the chip, or where the last tile would be mostly
   // empty.  Runs stay at 32 bytes or more.
@@ -659,30 +669,59 @@ static bool line_setup(Plan& p, PassPlan& pp) {
   const bool moved = !b.jf_in || !b.jf_out;
   const int64_t run = moved ? 128 / elt : 1, run_min = moved ? 32 / elt : 1;
   const int64_t least = a.pair_real && !a.r2r_cplx ? 2 : 1;
-  int64_t T = std::max(run, least);
-  while (T < 64 && threads(lines(T)) < 256) T *= 2;
-  int64_t cap = 1;
-  while (cap < a.ldim[0]) cap *= 2;
-  T = std::min(T, std::max(cap, least));
-  while (T > least && (threads(lines(T)) > max_threads || bytes(lines(T)) > 80 * 1024)) T /= 2;
   auto tiles = [&](int64_t t) {
     int64_t n = ceil_div(a.ldim[0], t);
     for (int i = 1; i < a.D; ++i) n *= a.ldim[i];
     return n;
   };
-  while (T > std::max(run_min, least) && T > least &&
-         (tiles(T) < 1024 || (a.ldim[0] * 5 < ceil_div(a.ldim[0], T) * T * 4)) &&
-         threads(lines(T)) > 64)
-    T /= 2;
+  int64_t cap = 1;
+  while (cap < a.ldim[0]) cap *= 2;
+  auto fits = [&](int64_t t) {
+    return threads(lines(t)) <= max_threads && bytes(lines(t)) <= 80 * 1024;
+  };
+  auto tile = [&](int64_t grid) {
+    int64_t t = std::max(run, least);
+    while (t < 64 && threads(lines(t)) < 256) t *= 2;
+    while (t < 64 && threads(lines(2 * t)) == threads(lines(t)) && fits(2 * t)) t *= 2;
+    t = std::min(t, std::max(cap, least));
+    while (t > least && !fits(t)) t /= 2;
+    while (t > std::max(run_min, least) && threads(lines(t / 2)) < threads(lines(t)) &&
+           (tiles(t) < grid || (a.ldim[0] * 5 < ceil_div(a.ldim[0], t) * t * 4)))
+      t /= 2;
+    return t;
+  };
+  int64_t T = tile(1024);
+  // Arrays that leave most of the chip idle: the time is that of one wavefront's
+  // instructions, so one butterfly a thread, of radices that keep them few
+  // (below half of the 1024 threads a CU holds at 4 wavefronts per SIMD).
+  if (b.form == LF_DIRECT && tiles(T) * threads(lines(T)) < kLineSmallThreads) {
+    b.form = LF_SMALL;
+    pts = 1;
+    S = line_schedule(M, rad, true);
+    T = tile(512);
+  }
+  b.S = S;
   const int64_t Tw = lines(T);
-  if (threads(Tw) > max_threads || bytes(Tw) > kMaxLds || reach(T) >= ((int64_t)1 << 31))
+  if (threads(Tw) > max_threads || bytes(Tw) > kMaxLds || reach(T) >= ((int64_t)1 << 31) ||
+      tiles(T) >= ((int64_t)1 << 31))
     return false;
   b.threads = (uint32_t)threads(Tw);
+  // The load and store loops of the R2R kinds, on such arrays, in one round of
+  // four points a thread (420 x 56 x 60 Float32, 56-point RODFT11 pass: 30.9 us
+  // with the stages' threads, 28.3 us; a prime's stage bounds the lines that have one)
+  if (b.form == LF_PRIME && rad[0] <= 16 && tiles(T) * threads(Tw) < kLineSmallThreads)
+    b.threads = (uint32_t)std::max(threads(Tw), std::min(max_threads, ceil_div(Tw * M, 256) * 64));
   b.Tw = (uint32_t)Tw;
   while (((int64_t)1 << b.twlog) < Tw) ++b.twlog;
   b.pitch = (uint32_t)pitch(Tw);
   b.m_half = reciprocal(a.M / 2 + 1);
   b.m_line = reciprocal(a.M);
+  auto reciprocal64 = [](int64_t d) -> uint64_t {   // ceil(2^64 / d)
+    return d <= 1 ? 0 : ~(uint64_t)0 / (uint64_t)d + 1;
+  };
+  b.blocks = (uint32_t)ceil_div(a.ldim[0], T);
+  b.m_blocks = reciprocal64(b.blocks);
+  for (int i = 1; i < a.D; ++i) b.m_dim[i] = reciprocal64(a.ldim[i]);
   // Stages and their twiddles: entries of the M-point table in the order the
   // kernel reads them (Bluestein: of the convolution's FFTs, decimation in
   // frequency, ns the distance of a butterfly's points).
