@@ -19,6 +19,22 @@ _TORCH_DTYPES = {L.F32: torch.float32, L.F64: torch.float64,
 _NAMES = Tr.ELTYPE_NAMES
 
 
+# The raw handle of a device's current stream: what the C calls take.  Small
+# transforms are bound by the host (64^3 Float64: six launches of 3.5 us in the
+# HIP runtime and the calls' own checks), and a torch.cuda.Stream object made
+# for each call costs 2 us of it.
+_raw_current_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _stream_handle(stream, tensor):
+    """The HIP stream of a call: `stream`, or the current one of the tensor's device."""
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_current_stream is not None:
+        return _raw_current_stream(tensor.get_device())
+    return torch.cuda.current_stream(tensor.device).cuda_stream
+
+
 def _real_type_code(t):
     if t in (L.F32, L.F64):
         return t
@@ -42,9 +58,10 @@ class Pencil:
         return tuple(self.size_global[p - 1] for p in self.permutation) + self.extra_dims
 
     def __eq__(self, other):
-        return (isinstance(other, Pencil) and self.size_global == other.size_global
-                and self.permutation == other.permutation
-                and self.extra_dims == other.extra_dims)
+        return self is other or (
+            isinstance(other, Pencil) and self.size_global == other.size_global
+            and self.permutation == other.permutation
+            and self.extra_dims == other.extra_dims)
 
     def __repr__(self):
         return "Pencil(size_global=%s, permutation=%s, extra_dims=%s)" % (
@@ -147,8 +164,9 @@ class ManyPencilArray:
 
 
 def _mightalias(a, b):
-    pa, pb = a.data_ptr(), b.data_ptr()
-    return pa < pb + b.nbytes() and pb < pa + a.nbytes()
+    ta, tb = a.parent, b.parent
+    pa, pb = ta.data_ptr(), tb.data_ptr()
+    return pa < pb + tb.nbytes and pb < pa + ta.nbytes
 
 
 class PencilFFTPlan:
@@ -312,19 +330,18 @@ class PencilFFTPlan:
 
     def _check_arrays(self, inp, out, inp_pencil, out_pencil, inp_type, out_type):
         # operations.jl:87-127
-        for a in (inp, out):
-            if not isinstance(a, PencilArray):
-                raise L.ArgumentError(L.ERR_ARGUMENT, "array types (%s, %s) incompatible with "
-                                      "out-of-place plans" % (type(inp).__name__,
-                                                              type(out).__name__))
+        if not (isinstance(inp, PencilArray) and isinstance(out, PencilArray)):
+            raise L.ArgumentError(L.ERR_ARGUMENT, "array types (%s, %s) incompatible with "
+                                  "out-of-place plans" % (type(inp).__name__,
+                                                          type(out).__name__))
         if _mightalias(inp, out):
             raise L.ArgumentError(L.ERR_ARGUMENT, "out-of-place plan applied to aliased data")
         if inp.pencil != inp_pencil or inp.eltype != inp_type:
             raise L.ArgumentError(L.ERR_ARGUMENT, "unexpected dimensions of input data")
         if out.pencil != out_pencil or out.eltype != out_type:
             raise L.ArgumentError(L.ERR_ARGUMENT, "unexpected dimensions of output data")
-        for a in (inp, out):
-            if not a.parent.is_cuda or not a.parent.is_contiguous():
+        for t in (inp.parent, out.parent):
+            if not t.is_cuda or not t.is_contiguous():
                 raise L.ArgumentError(L.ERR_ARGUMENT,
                                       "arrays must be contiguous GPU tensors")
 
@@ -341,19 +358,20 @@ class PencilFFTPlan:
         else:
             self._check_arrays(src, dst, self.pencil_output, self.pencil_input,
                                self.eltype_output, self.eltype_input)
-        s = stream if stream is not None else torch.cuda.current_stream(src.parent.device)
-        self._launch(direction, src.data_ptr(), dst.data_ptr(), s, op)
+        self._launch(direction, src.parent.data_ptr(), dst.parent.data_ptr(),
+                     _stream_handle(stream, src.parent), op)
         return dst
 
-    def _launch(self, direction, pin, pout, s, op):
+    def _launch(self, direction, pin, pout, stream, op):
         w = self._workspace()
         wp = w.data_ptr() if w is not None else None
         if op is None:
-            L.check(L.lib.pfft_execute(self._h, direction, pin, pout, wp, self.work_bytes,
-                                       s.cuda_stream))
+            status = L.lib.pfft_execute(self._h, direction, pin, pout, wp, self.work_bytes, stream)
         else:
-            L.check(L.lib.pfft_execute_op(self._h, direction, C.byref(op), pin, pout, wp,
-                                          self.work_bytes, s.cuda_stream))
+            status = L.lib.pfft_execute_op(self._h, direction, C.byref(op), pin, pout, wp,
+                                           self.work_bytes, stream)
+        if status:
+            L.check(status)
 
     def _execute_inplace(self, direction, src, dst, stream=None, op=None):
         # operations.jl:100-116: the same ManyPencilArray in and out
@@ -369,8 +387,8 @@ class PencilFFTPlan:
             raise L.ArgumentError(L.ERR_ARGUMENT, "unexpected dimensions of output data")
         if src.nbytes() < self.in_bytes or not src.data.is_cuda:
             raise L.ArgumentError(L.ERR_ARGUMENT, "buffer too small for the in-place plan")
-        s = stream if stream is not None else torch.cuda.current_stream(src.data.device)
-        self._launch(direction, src.data_ptr(), src.data_ptr(), s, op)
+        ptr = src.data_ptr()
+        self._launch(direction, ptr, ptr, _stream_handle(stream, src.data), op)
         return dst
 
     def _maybe_allocate(self, allocator, src):
@@ -548,8 +566,8 @@ def execute_batch(items, stream=None):
         arr[k].out = dst.data_ptr()
         arr[k].work = w.data_ptr() if w is not None else None
         arr[k].work_bytes = p.work_bytes
-    s = stream if stream is not None else torch.cuda.current_stream(items[0][2].parent.device)
-    L.check(L.lib.pfft_execute_batch(len(items), arr, s.cuda_stream))
+    L.check(L.lib.pfft_execute_batch(len(items), arr,
+                                     _stream_handle(stream, items[0][2].parent)))
 
 
 def execute_many(direction, p, dsts, srcs):
@@ -567,8 +585,7 @@ def execute_many(direction, p, dsts, srcs):
     ins = (C.c_void_p * n)(*[s.data_ptr() for s in srcs])
     outs = (C.c_void_p * n)(*[d.data_ptr() for d in dsts])
     w = p._workspace()
-    st = torch.cuda.current_stream(srcs[0].parent.device)
     L.check(L.lib.pfft_execute_many(p._h, direction, n, ins, outs,
                                     w.data_ptr() if w is not None else None, p.work_bytes,
-                                    st.cuda_stream))
+                                    _stream_handle(None, srcs[0].parent)))
     return dsts

@@ -91,7 +91,7 @@ def project_divergence_free_(uhs, p, scale=None, stream=None):
     """In place: uh_i <- uh_i - k_i (k . uh) / |k|^2 on the three output-shaped
     spectra uhs (docs/examples/navier_stokes.jl:351-366); the mean mode is
     left as is.  One elementwise kernel (pfft_project_divergence_free)."""
-    import torch
+    from .plans import _stream_handle
     if len(uhs) != 3:
         raise L.ArgumentError(L.ERR_ARGUMENT,
                               "the divergence-free projection takes three components")
@@ -99,7 +99,6 @@ def project_divergence_free_(uhs, p, scale=None, stream=None):
         if a.pencil != p.pencil_output or a.eltype != p.eltype_output:
             raise L.ArgumentError(L.ERR_ARGUMENT, "unexpected dimensions of input/output data")
     sc = (C.c_double * 3)(*scale) if scale is not None else None
-    s = stream if stream is not None else torch.cuda.current_stream(uhs[0].parent.device)
     L.check(L.lib.pfft_project_divergence_free(p._h, *(a.data_ptr() for a in uhs), sc,
-                                               s.cuda_stream))
+                                               _stream_handle(stream, uhs[0].parent)))
     return uhs
