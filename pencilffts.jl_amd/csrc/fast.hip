@@ -37,6 +37,7 @@
 #include "../../include/pfft.h"
 #include "fast_pass.hpp"
 #include "generic_pass.hpp"
+#include "touch_args.hpp"
 
 namespace pfft {
 namespace fk {
@@ -1053,6 +1054,7 @@ __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1))) void k_fast(PassArgs a) 
   constexpr bool POST =
       (KIND == K_R2C || DCTLIKE || KIND == K_DHTC) && !ROWPERM;   // post reads LDS
   constexpr int NX = KIND == K_R2C ? P + 1 : P;   // outputs per lane per line
+  touch_args<sizeof(PassArgs)>();
   extern __shared__ __align__(16) char smem[];
   C<R>* lds = (C<R>*)smem;
   const int tid = threadIdx.x;

@@ -162,8 +162,9 @@ PFFT_HD void tile_init(const PassArgs& a, int64_t tile, TileCtx& c) {
   int64_t ib = b0 * a.T * a.lsin[0];
   int64_t ob = b0 * a.T * a.lsout[0];
   for (int d = 1; d < a.D; ++d) {
-    const int64_t m = rest % a.ldim[d];
-    rest /= a.ldim[d];
+    const int64_t q = d + 1 < a.D ? rest / a.ldim[d] : 0;   // (nothing past the last dim)
+    const int64_t m = rest - q * a.ldim[d];
+    rest = q;
     ib += m * a.lsin[d];
     ob += m * a.lsout[d];
   }

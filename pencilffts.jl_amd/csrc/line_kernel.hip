@@ -8,6 +8,7 @@
 
 #include "line_prime.hpp"
 #include "plan.hpp"
+#include "touch_args.hpp"
 
 #define PFFT_CAT3_(a, b, c) a##b##c
 #define PFFT_CAT3(a, b, c) PFFT_CAT3_(a, b, c)
@@ -23,28 +24,12 @@ __device__ __forceinline__ uint32_t opaque(uint32_t x) {
   return x;
 }
 
-// Touches every cache line of the kernel's arguments at once.  Read where they
-// are first needed they miss one after the other, each miss a trip to the
-// memory the host wrote them to: the first global load of a pass then left
-// 1.8 us after the wavefront started, half the time of a pass on a small array
-// (0.9 us with this, the reciprocals of line_tile and opaque_s).
-__device__ __forceinline__ void touch_args() {
-  static_assert(sizeof(PassArgs) + sizeof(LineArgs) > 15 * 64 &&
-                    sizeof(PassArgs) + sizeof(LineArgs) <= 16 * 64,
-                "one word of each 64 bytes");
-  const auto* k = (const __attribute__((address_space(4))) uint32_t*)
-      __builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" ::"s"(k[0]), "s"(k[16]), "s"(k[32]), "s"(k[48]), "s"(k[64]), "s"(k[80]),
-               "s"(k[96]), "s"(k[112]), "s"(k[128]), "s"(k[144]), "s"(k[160]), "s"(k[176]),
-               "s"(k[192]), "s"(k[208]), "s"(k[224]), "s"(k[240]));
-}
-
 #if PFFT_LINE_FORM == 1
 // (float: held to 128 VGPRs, 4 waves per SIMD; it asks for 130)
 template <typename R, int CLS>
 __global__ __launch_bounds__(line_max_threads(CLS, LF_BLUESTEIN, sizeof(R) == 4),
                              sizeof(R) == 4 ? 4 : 2) void k_line_bs(PassArgs a, LineArgs b) {
-  touch_args();
+  touch_args<sizeof(PassArgs) + sizeof(LineArgs)>();
   extern __shared__ __align__(16) char lds[];
   cpx<R>* W = (cpx<R>*)lds;
   const uint32_t tid = threadIdx.x;
@@ -83,7 +68,7 @@ __global__ __launch_bounds__(line_max_threads(CLS, LF_BLUESTEIN, sizeof(R) == 4)
 #elif PFFT_LINE_FORM == 2
 template <typename R, int CLS>
 __global__ __launch_bounds__(kLineMaxThreads) void k_line_prime(PassArgs a, LineArgs b) {
-  touch_args();
+  touch_args<sizeof(PassArgs) + sizeof(LineArgs)>();
   extern __shared__ __align__(16) char lds[];
   cpx<R>* W = (cpx<R>*)lds;
   const uint32_t tid = threadIdx.x;
@@ -124,7 +109,7 @@ __global__ __launch_bounds__(kLineMaxThreads) void k_line_prime(PassArgs a, Line
 #else
 template <typename R, int CLS, int PTS>
 __global__ __launch_bounds__(kLineMaxThreads) void k_line(PassArgs a, LineArgs b) {
-  touch_args();
+  touch_args<sizeof(PassArgs) + sizeof(LineArgs)>();
   extern __shared__ __align__(16) char lds[];
   cpx<R>* W = (cpx<R>*)lds;
   const uint32_t tid = threadIdx.x;
