@@ -37,6 +37,8 @@ LINE_OBJECTS = [("line_%s_%s%d.o" % (name, form, c),
                 for c in reversed(range(LINE_CLASSES)) for k, form in enumerate(("", "bs", "prime", "small"))
                 for real, name in (("double", "f64"), ("float", "f32"))
                 if not (c == 5 and form in ("", "small"))]   # (R2R: no direct forms)
+PLANE_OBJECTS = [("plane_%s.o" % name, ["-DPFFT_PLANE_REAL=" + real, "-DPFFT_PLANE_NAME=" + name])
+                 for real, name in (("double", "f64"), ("float", "f32"))]
 EMU_SOURCES = ["emu.cpp", "plan.cpp"]
 
 
@@ -64,11 +66,12 @@ def build(verbose=False):
         dev = DEVICE_FLAGS if src.endswith(".hip") else []
         jobs.append([HIPCC] + COMMON + dev + lang + ["-c", os.path.join(CSRC, src), "-o", obj])
         objs.append(obj)
-    for name, defines in LINE_OBJECTS:
-        obj = os.path.join(LIB, name)
-        jobs.append([HIPCC] + COMMON + DEVICE_FLAGS + defines +
-                    ["-x", "hip", "-c", os.path.join(CSRC, "line_kernel.hip"), "-o", obj])
-        objs.append(obj)
+    for src, variants in (("plane_kernel.hip", PLANE_OBJECTS), ("line_kernel.hip", LINE_OBJECTS)):
+        for name, defines in variants:
+            obj = os.path.join(LIB, name)
+            jobs.append([HIPCC] + COMMON + DEVICE_FLAGS + defines +
+                        ["-x", "hip", "-c", os.path.join(CSRC, src), "-o", obj])
+            objs.append(obj)
     # host emulator (tests only): host compilation of the same phase functions
     for src in EMU_SOURCES:
         obj = os.path.join(LIB, "emu_" + src.replace(".", "_") + ".o")

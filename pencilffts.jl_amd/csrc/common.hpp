@@ -172,6 +172,24 @@ struct LineArgs {
   LineStage st[kLineStages];
 };
 
+// ---- plane pass (plane_pass.hpp) ----------------------------------------------
+// The first two dims of a 3D transform in one launch: x lines (ny of them) and
+// y lines (nx of them: the points x is stored in) of one plane per workgroup.
+struct PlaneDim {
+  int32_t S, bwd;
+  uint32_t lines, m_lines;   // lines of a plane, reciprocal
+  LineStage st[kLineStages]; // twiddles in PlaneArgs::tw
+};
+struct PlaneArgs {
+  int32_t on, fwd, cls;      // fwd: x then y; cls: LineClass of the x lines
+  uint32_t threads, pitch, sh;   // LDS: element (x, y) at y pitch + wp(x)
+  uint32_t m_pairs;          // reciprocal of the x lines' M / 2 + 1
+  int64_t sx_in, sy_in, sx_out, sy_out;   // element strides within a plane
+  uint64_t m_dim[kMaxDims];  // reciprocals of the plane dims (line_div64)
+  const void* tw;
+  PlaneDim x, y;
+};
+
 template <typename R>
 struct cpx {
   R re, im;

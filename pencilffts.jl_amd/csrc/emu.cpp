@@ -13,6 +13,7 @@
 #include "../../include/pfft.h"
 #include "generic_pass.hpp"
 #include "line_prime.hpp"
+#include "plane_pass.hpp"
 #include "plan.hpp"
 
 using namespace pfft;
@@ -169,8 +170,76 @@ static void emu_form(const PassPlan& pp, const PassArgs& a, const LineArgs& b) {
   }
 }
 
+template <typename R, int CLS, bool FWD>
+static void emu_plane(const PassPlan& pp, const PassArgs& a, const PlaneArgs& p) {
+  const int nthr = (int)p.threads;
+  std::vector<char> store((size_t)pp.lds_bytes + 16);
+  char* lds = store.data() + (16 - (size_t)store.data() % 16) % 16;
+  cpx<R>* W = (cpx<R>*)lds;
+  std::vector<cpx<R>> regs((size_t)nthr * kLinePoints);
+  auto v = [&](int t) { return &regs[(size_t)t * kLinePoints]; };
+  const PlaneDim& d0 = FWD ? p.x : p.y;
+  const PlaneDim& d1 = FWD ? p.y : p.x;
+  for (int64_t tile = 0; tile < a.ntiles; ++tile) {
+    TileCtx c;
+    plane_tile(a, p, (uint32_t)tile, c);
+    for (int s = 0; s < d0.S; ++s) {
+      for (int t = 0; t < nthr; ++t) {
+        if (s == 0) {
+#define PFFT_F(RAD) plane_load<R, CLS, FWD, RAD>(a, p, c, t, v(t))
+          PFFT_LINE_RADIX(d0.st[s].rad, PFFT_F)
+#undef PFFT_F
+        } else {
+#define PFFT_F(RAD) plane_get<R, !FWD, RAD>(p, d0, s, t, v(t), W)
+          PFFT_LINE_RADIX(d0.st[s].rad, PFFT_F)
+#undef PFFT_F
+        }
+      }
+      for (int t = 0; t < nthr; ++t) {
+#define PFFT_F(RAD) plane_put<R, !FWD, RAD>(p, d0, s, t, v(t), W)
+        PFFT_LINE_RADIX(d0.st[s].rad, PFFT_F)
+#undef PFFT_F
+      }
+    }
+    if (plane_has_middle(CLS))
+      for (int t = 0; t < nthr; ++t) plane_middle<R, CLS>(a, p, t, W);
+    for (int s = 0; s < d1.S; ++s) {
+      for (int t = 0; t < nthr; ++t) {
+#define PFFT_F(RAD) plane_get<R, FWD, RAD>(p, d1, s, t, v(t), W)
+        PFFT_LINE_RADIX(d1.st[s].rad, PFFT_F)
+#undef PFFT_F
+      }
+      for (int t = 0; t < nthr; ++t) {
+        if (s == d1.S - 1) {
+#define PFFT_F(RAD) plane_store<R, CLS, FWD, RAD>(a, p, c, t, v(t))
+          PFFT_LINE_RADIX(d1.st[s].rad, PFFT_F)
+#undef PFFT_F
+        } else {
+#define PFFT_F(RAD) plane_put<R, FWD, RAD>(p, d1, s, t, v(t), W)
+          PFFT_LINE_RADIX(d1.st[s].rad, PFFT_F)
+#undef PFFT_F
+        }
+      }
+    }
+  }
+}
+
 template <typename R>
 static void emu_any(const Plan& p, const PassPlan& pp, const PassArgs& a) {
+  if (pp.plane.on) {
+    PlaneArgs q = pp.plane;
+    q.tw = table_at(p, pp.line_tw_id, true);
+    switch (q.cls) {
+      case LC_R2C: emu_plane<R, LC_R2C, true>(pp, a, q); break;
+      case LC_R2C_ODD: emu_plane<R, LC_R2C_ODD, true>(pp, a, q); break;
+      case LC_C2R: emu_plane<R, LC_C2R, false>(pp, a, q); break;
+      case LC_C2R_ODD: emu_plane<R, LC_C2R_ODD, false>(pp, a, q); break;
+      default:
+        if (q.fwd) emu_plane<R, LC_C2C, true>(pp, a, q);
+        else emu_plane<R, LC_C2C, false>(pp, a, q);
+    }
+    return;
+  }
   if (!pp.line.S) {
     emu_pass<R>(pp, a);
     return;
@@ -195,8 +264,10 @@ __attribute__((visibility("default"))) int pfft_emu_plan_create(
     int32_t real_type, int32_t permute, int32_t n_extra, const int64_t* extra, uint32_t flags) {
   *out = nullptr;
   pfft_emu_plan* h = new pfft_emu_plan();
-  int r = plan_build(h->p, ndims, dims, kinds, real_type, permute, n_extra, extra,
-                     flags | PFFT_FLAG_GENERIC_ONLY);
+  // bit 31 lets plans fuse their first two dims (the emulator's plans are
+  // otherwise chains of single passes)
+  const uint32_t fl = flags >> 31 ? flags & 0x7fffffffu : flags | PFFT_FLAG_GENERIC_ONLY;
+  int r = plan_build(h->p, ndims, dims, kinds, real_type, permute, n_extra, extra, fl);
   if (r) {
     delete h;
     return r;

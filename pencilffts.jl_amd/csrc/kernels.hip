@@ -114,10 +114,20 @@ static int line_prepare(const Plan& p, const PassPlan& pp) {
   return r;
 }
 
-// the general kernel of a pass: the line pass, or the phases of the generic one
+// the kernels of the plane pass (plane_kernel.hip)
+int plane_prepare_f32(const PassPlan& pp);
+int plane_prepare_f64(const PassPlan& pp);
+void plane_launch_f32(const PassPlan& pp, const PassArgs& a, const PlaneArgs& p, hipStream_t st);
+void plane_launch_f64(const PassPlan& pp, const PassArgs& a, const PlaneArgs& p, hipStream_t st);
+
+// the general kernel of a pass: a plane or line pass, or the phases of the generic one
 static void launch_generic(const Plan& p, const PassPlan& pp, const PassArgs& a,
                            hipStream_t st) {
-  if (pp.line.S) {
+  if (pp.plane.on) {
+    PlaneArgs q = pp.plane;
+    q.tw = table_at(p, pp.line_tw_id);
+    (p.real_type == PFFT_F32 ? plane_launch_f32 : plane_launch_f64)(pp, a, q, st);
+  } else if (pp.line.S) {
     LineArgs b = pp.line;
     b.tw = table_at(p, pp.line_tw_id);
     const int cls = b.cls == LC_C2C && (a.op || a.fs_M) ? (int)LC_C2C_OP : b.cls;
@@ -280,6 +290,7 @@ static int launch_pass(const Plan& p, const PassPlan& pp, const void* src, void*
 
 static int prepare_pass(const Plan& p, const PassPlan& pp) {
   if (pp.variant != 0) return fast_prepare(pp);
+  if (pp.plane.on) return p.real_type == PFFT_F32 ? plane_prepare_f32(pp) : plane_prepare_f64(pp);
   if (pp.line.S) return line_prepare(p, pp);
   return set_lds_limit(generic_fn(p.real_type, pp), pp.lds_bytes);
 }
@@ -530,6 +541,7 @@ static int autotune(Plan& p) {
   };
   auto consider = [&](PassPlan& pp, const PassPlan& base, int op_side, const PassPlan* prod,
                       int list, int index) {
+    if (base.plane.on) return;
     std::vector<int> c = fast_candidates(p, base, op_side != 0);
     if (c.empty()) return;
     const int rev = ((p.flags & PFFT_FLAG_REVERSE_TILES) ? kVariantReverse : 0) |
@@ -874,7 +886,9 @@ int device_pass_names(Plan& p, int dir, std::string* out) {
   for (size_t i = 0; i < passes.size(); ++i) {
     if (i) *out += ";";
     *out += passes[i].variant == 0
-                ? std::string(passes[i].line.S ? "k_line" : "k_generic") +
+                ? std::string(passes[i].plane.on ? "k_plane"
+                              : passes[i].line.S ? "k_line"
+                                                 : "k_generic") +
                       (p.real_type == PFFT_F32 ? "<f32>" : "<f64>")
                 : std::string(fast_name(passes[i].variant));
     if (passes[i].variant == 0 && passes[i].args.bs_M)

@@ -8,6 +8,7 @@
 // and then lowers every stage to one fused pass (transform + the transpose
 // into the next pencil's memory order).
 #include "plan.hpp"
+#include "plane_pass.hpp"
 
 #include <math.h>
 #include <string.h>
@@ -1071,6 +1072,167 @@ static int build_pass(Plan& p, int dim, int32_t kind, int32_t elt_in, int32_t el
   return PFFT_OK;
 }
 
+// ---- plane pass (plane_pass.hpp) -----------------------------------------------
+// Whether a plane pass is the better one: planes of X x Y points in LDS, `planes`
+// of them, a workgroup each.  It saves a launch each way (a pair of calls is 23-25 us
+// of host time in six launches, 17-18 in four) and gives up parallelism: a
+// plane's work runs on one CU.
+//   Small planes of small arrays, any length: 16 x 32 x 64 Float64 r2c pairs 25.6
+//   -> 22.7 us, 32^3 26.8 -> 23.5, 32 x 32 x 256 complex 30.8 -> 28.2; past it 64^3
+//   27.9 -> 31.6 us, 32 x 32 x 4096 147 -> 202.
+//   Lengths the specialised kernels lack (odd part above 3) take the line pass, which
+//   a plane pass also beats with more points, while the planes are not few: r2c
+//   pairs of 40^3 Float64 30.0 -> 26.6 us, 90^3 55.6 -> 45.4, 100^3 63.2 -> 53.2; past
+//   it 110 x 110 x 50 Float32 37.1 -> 38.1, 180 x 120 x 60 47.3 -> 50.0.
+static bool plane_fits(int64_t X, int64_t Y, int64_t n, int64_t planes) {
+  auto odd_part = [](int64_t k) { while (k % 2 == 0) k /= 2; return k; };
+  if (X * Y <= 1088 && X * Y * planes <= 1 << 18) return true;
+  return (odd_part(n) > 3 || odd_part(Y) > 3) && X * Y <= 8192 && planes <= 256 &&
+         planes * 100 >= X * Y;
+}
+
+// Stages of one dim of a plane pass; their twiddles are appended to `tw`.  False
+// where the length has no register radices or a stage's butterflies do not
+// fit the threads.
+static bool plane_dim(Plan& p, int64_t M, int64_t lines, bool bwd, int64_t max_threads,
+                      PlaneDim* d, std::vector<double>* tw, int64_t* threads) {
+  int32_t rad[kLineStages];
+  for (bool small : {true, false}) {
+    const int S = line_schedule(M, rad, small);
+    if (!S || rad[0] > 16) return false;
+    // one butterfly a thread where the workgroup is large enough for it
+    int64_t want = 0;
+    bool ok = true;
+    for (int s = 0; s < S; ++s) {
+      const int64_t n = lines * (M / rad[s]);
+      want = std::max(want, std::min(max_threads, ceil_div(n, 64) * 64));
+      ok = ok && ceil_div(n, max_threads) <= line_bpt(rad[s]);
+    }
+    if (!ok) continue;
+    d->S = S;
+    d->bwd = bwd;
+    d->lines = (uint32_t)lines;
+    d->m_lines = reciprocal(lines);
+    *threads = std::max(*threads, want);
+    const std::vector<double> w = p.tables[twiddle_table(p, M)].values;
+    int64_t ns = 1;
+    for (int s = 0; s < S; ++s) {
+      LineStage& st = d->st[s];
+      st.rad = (uint32_t)rad[s];
+      st.nb = (uint32_t)(M / rad[s]);
+      st.ns = (uint32_t)ns;
+      st.m_nb = reciprocal(st.nb);
+      st.m_ns = reciprocal(ns);
+      st.tw = (uint32_t)(tw->size() / 2);
+      const int64_t step = M / (ns * rad[s]);
+      if (s)
+        for (int64_t r = 1; r < rad[s]; ++r)
+          for (int64_t jj = 0; jj < ns; ++jj) {
+            const size_t k = 2 * (size_t)(r * jj * step);
+            tw->push_back(w[k]);
+            tw->push_back(w[k + 1]);
+          }
+      ns *= rad[s];
+    }
+    return true;
+  }
+  return false;
+}
+
+// The pass over dims 0 and 1 of a 3D out-of-place plan (fwd: from the input
+// pencil, else into it), the other side in natural order; false where it does
+// not apply.
+static bool plane_pass(Plan& p, bool fwd, PassPlan* out) {
+  const Stage &sx = p.stages[0], &sy = p.stages[1];
+  const int32_t kx = kind_base(fwd ? sx.kind_fwd : sx.kind_bwd);
+  const int32_t ky = kind_base(fwd ? sy.kind_fwd : sy.kind_bwd);
+  if (!is_c2c(ky)) return false;
+  PassPlan pp;
+  PassArgs& a = pp.args;
+  memset(&a, 0, sizeof(a));
+  const int64_t nx = p.size_in[0], mx = p.size_out[0], Y = p.size_in[1];
+  a.n = nx;
+  a.M = nx;
+  a.kind = L_C2C;
+  if (fwd ? kx == PFFT_RFFT : is_c2r(kx)) {
+    const bool even = nx % 2 == 0;
+    a.kind = fwd ? (even ? L_R2C_HALF : L_R2C_FULL) : (even ? L_C2R_HALF : L_C2R_FULL);
+    if (even) a.M = nx / 2;
+  } else if (!is_c2c(kx)) {
+    return false;
+  }
+  if (a.M < 2 || Y < 2 || largest_prime_factor(a.M) > 13 || largest_prime_factor(Y) > 13)
+    return false;
+  a.bwd = kx == PFFT_BFFT || is_c2r(kx);
+  pp.elt_in = fwd ? sx.elt_in : sy.elt_out;
+  pp.elt_out = fwd ? sy.elt_out : sx.elt_in;
+  a.in_cplx = eltype_is_complex(pp.elt_in);
+  a.out_cplx = eltype_is_complex(pp.elt_out);
+  const bool f32 = p.real_type == PFFT_F32;
+  const int64_t rs = f32 ? 4 : 8, cs = 2 * rs;
+  PlaneArgs& q = pp.plane;
+  q.on = 1;
+  q.fwd = fwd;
+  q.cls = line_class(a.kind);
+  // the plane in LDS: rows of the longer of the stored and the transformed line
+  const int64_t row = std::max(a.M, mx);
+  q.sh = f32 ? 5 : 4;
+  q.pitch = (uint32_t)((row + ((row - 1) >> q.sh)) | 1);
+  pp.lds_bytes = Y * (int64_t)q.pitch * cs;
+  if (pp.lds_bytes > kMaxLds) return false;
+  const int64_t planes = p.size_in[2] * p.E;
+  if (planes >= ((int64_t)1 << 31) || !plane_fits(mx, Y, nx, planes) ||
+      Y * cs >= 2048 || p.size_in[2] * cs >= 8192) return false;
+  pp.tw_id = pp.aux_id = -1;
+  pp.variant = 0;
+  std::vector<double> tw;
+  int64_t threads = 0;
+  if (!plane_dim(p, a.M, Y, a.bwd != 0, plane_max_threads(f32), &q.x, &tw, &threads) ||
+      !plane_dim(p, Y, mx, ky == PFFT_BFFT, plane_max_threads(f32), &q.y, &tw, &threads) ||
+      line_fft(p, pp, false) != PFFT_OK)
+    return false;
+  q.threads = (uint32_t)threads;
+  q.m_pairs = reciprocal(a.M / 2 + 1);
+  if (!tw.empty()) {
+    std::string key = "plane";
+    for (const PlaneDim* d : {&q.x, &q.y})
+      for (int s = 0; s < d->S; ++s) key += "," + std::to_string(d->st[s].rad);
+    pp.line_tw_id = find_table(p, key);
+    if (pp.line_tw_id < 0) pp.line_tw_id = add_table(p, key, std::move(tw));
+  }
+  const int64_t in_x = fwd ? nx : mx, out_x = fwd ? mx : nx;
+  q.sx_in = q.sx_out = 1;
+  q.sy_in = in_x;
+  q.sy_out = out_x;
+  a.L_in = in_x;
+  a.L_out = out_x;
+  a.sk_in = a.sk_out = 1;
+  a.T = 1;
+  a.D = p.E > 1 ? 2 : 1;
+  a.ldim[0] = p.size_in[2];
+  a.lsin[0] = in_x * Y;
+  a.lsout[0] = out_x * Y;
+  a.llog[0] = 2;
+  a.ldim[1] = p.E;
+  a.lsin[1] = a.lsin[0] * p.size_in[2];
+  a.lsout[1] = a.lsout[0] * p.size_in[2];
+  a.llog[1] = -1;
+  for (int d = 0; d < a.D; ++d)
+    q.m_dim[d] = a.ldim[d] <= 1 ? 0 : ~(uint64_t)0 / (uint64_t)a.ldim[d] + 1;
+  a.scale = 1.0;
+  a.ntiles = planes;
+  pp.in_elems = planes * in_x * Y;
+  pp.out_elems = planes * out_x * Y;
+  pp.grid = std::min<int64_t>(planes, 1 << 20);
+  pp.threads = (int32_t)threads;
+  pp.gen_args = a;
+  pp.gen_threads = pp.threads;
+  pp.gen_lds = pp.lds_bytes;
+  pp.gen_grid = pp.grid;
+  *out = pp;
+  return true;
+}
+
 // ---- spectral operators (pfft_execute_op) ------------------------------------
 int op_setup(const Plan& p, int dir, const pfft_spectral_op& op, int* pass, int* side) {
   if (op.op < PFFT_OP_DERIVATIVE || op.op > PFFT_OP_DEALIAS)
@@ -1270,7 +1432,26 @@ int plan_build(Plan& p, int32_t N, const int64_t* dims, const int32_t* kinds,
     if (row < (tile_load ? 2048 : 8192)) return 0;
     return len + 32;
   };
-  {
+  // The first two dims in one pass.  Not where a flag asks for particular kernels
+  // of the single passes.
+  const uint32_t single = PFFT_FLAG_GENERIC_ONLY | PFFT_FLAG_MFMA_SPLIT16 |
+                          PFFT_FLAG_MFMA_BF16X3 | PFFT_FLAG_REVERSE_TILES |
+                          PFFT_FLAG_STREAM_STORES | (0xffu << 16);
+  PassPlan plane_fwd, plane_bwd;
+  const bool planes = N == 3 && !p.inplace && !(p.flags & single) &&
+                      plane_pass(p, true, &plane_fwd) && plane_pass(p, false, &plane_bwd);
+  const int32_t natural[3] = {0, 1, 2};
+  if (planes) {
+    const Stage& s = p.stages[2];
+    p.fwd.push_back(plane_fwd);
+    int r = build_pass(p, 2, s.kind_fwd, s.elt_in, s.elt_out, natural, s.dims_before, s.perm,
+                       s.dims_after, p.fwd);
+    if (!r) r = build_pass(p, 2, s.kind_bwd, s.elt_out, s.elt_in, s.perm, s.dims_after, natural,
+                           s.dims_before, p.bwd);
+    if (r) return r;
+    p.bwd.push_back(plane_bwd);
+  }
+  if (!planes) {
     int32_t cur[kMaxDims];
     int64_t cur_pad = pad_real;
     memcpy(cur, p.stages[0].perm, sizeof(cur));
@@ -1288,7 +1469,7 @@ int plan_build(Plan& p, int32_t N, const int64_t* dims, const int32_t* kinds,
       cur_pad = pad_out;
     }
   }
-  {
+  if (!planes) {
     int32_t cur[kMaxDims];
     int64_t cur_pad = 0;
     memcpy(cur, p.stages[N - 1].perm, sizeof(cur));

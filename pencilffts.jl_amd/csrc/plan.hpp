@@ -64,6 +64,8 @@ struct PassPlan {
   // phases of the generic pass
   LineArgs line = {};
   int32_t line_tw_id = -1;  // index into Plan::tables (stage twiddles), -1 = none
+  // a plane pass where plane.on (args: the x lines', their line dims the planes)
+  PlaneArgs plane = {};
 };
 
 struct Table {

@@ -78,6 +78,20 @@ class Emulator:
         finally:
             self.lib.pfft_emu_plan_destroy(h)
 
+    def passes(self, dims, kinds, real_type, permute=True, extra=(), flags=0):
+        """Number of forward passes (launches) of the plan."""
+        N, ne = len(dims), len(extra)
+        h = C.c_void_p()
+        st = self.lib.pfft_emu_plan_create(
+            C.byref(h), N, (C.c_int64 * N)(*dims), (C.c_int32 * N)(*kinds), real_type,
+            int(permute), ne, (C.c_int64 * max(ne, 1))(*extra), flags)
+        if st:
+            raise RuntimeError(self.lib.pfft_emu_last_error().decode())
+        self.lib.pfft_emu_bluestein.restype = C.c_int
+        n = self.lib.pfft_emu_bluestein(h, (C.c_int64 * 16)(), 16)
+        self.lib.pfft_emu_plan_destroy(h)
+        return n
+
     def run_inplace(self, dims, kinds, real_type, directions, buf, permute=True, extra=()):
         """In-place plan: runs each direction in turn on the uint8 buffer `buf`
         (input and output views share it); returns the plan's buffer size."""
