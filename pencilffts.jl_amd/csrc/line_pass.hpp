@@ -21,9 +21,9 @@
 // lines masks the others: odd and ragged extents take the same path.
 //
 // What bounds it: HBM traffic on the two-stage lengths (180-point lines of
-// 240 x 200 x 180 complex doubles, 276 MB, in 52-60 us), latency between the
+// 240 x 200 x 180 complex doubles, 276 MB, in 48-53 us), latency between the
 // barriers with two workgroups on a CU on the three-stage ones (448-point lines
-// of 448 x 352 x 208 complex floats, 525 MB, in 130-150 us).  The generic
+// of 448 x 352 x 208 complex floats, 525 MB, in 123-128 us).  The generic
 // phases, with one trip through LDS and one barrier per radix of at most 8
 // and two more for loading and storing, took 119-167 and 303-343 us.  16
 // points a thread keep S low; 8 (radices to 8) cost one more trip.

@@ -12,7 +12,7 @@
 // device, 3.5 us of the host's): one launch of three and one trip through memory
 // less.  What bounds it: latency, of the launch, of one load of the plane and of two
 // barriers a stage, with as many CUs at work as there are planes.  Measured, pairs
-// of Float64 r2c plans called one by one: 16 x 32 x 64 27.0 -> 22.7 us, 28 x 28 x 12
+// of Float64 r2c plans called one by one (single passes -> plane pass): 16 x 32 x 64 27.0 -> 21.7 us, 28 x 28 x 12
 // 29.2 -> 22.2, 105 planes of 112 x 65 59.3 -> 50.6 (the rule, with both sides: plane_fits
 // in plan.cpp).
 //

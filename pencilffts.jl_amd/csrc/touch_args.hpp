@@ -11,8 +11,8 @@ namespace pfft {
 // Measured on the line pass: the first global load of a pass left 1.8 us after
 // the wavefront started, half the time of a pass on a small array (0.9 us with
 // this and reciprocals for the tile's divisions).  In the specialised kernels: pairs
-// of Float64 r2c plans 64^3 29.0 -> 27.7 us, 16 x 32 x 64 by single passes 29.2 -> 27.0,
-// 256^3 304 -> 299.
+// of Float64 r2c plans 64^3 29.0 -> 26.6 us, 16 x 32 x 64 by single passes 29.2 -> 27.0,
+// 256^3 304 -> 296.
 template <int BYTES>
 __device__ __forceinline__ void touch_args() {
   static_assert(BYTES <= 24 * 64, "one word of each 64 bytes");
